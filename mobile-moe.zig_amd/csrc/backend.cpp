@@ -264,7 +264,7 @@ int gemv_device(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t first, uint64_t 
         {
             TimedLaunch tl(ctx, "gemv_float");
             e = launch_gemv_float(base, w->type, mstride, x, x_stride, y, y_stride, (uint32_t)n, (uint32_t)w->rows,
-                                  (uint32_t)w->cols, ctx->stream);
+                                  (uint32_t)w->cols, ctx->num_cu, ctx->stream);
         }
         return e == hipSuccess ? MMHIP_OK : hip_fail(e, "gemv: launch");
     }
@@ -320,7 +320,7 @@ int qmm_device(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t mat, const float*
         const uint64_t es = (w->type == kF32) ? 4 : 2;
         const char* base = static_cast<const char*>(w->plain) + mat * w->rows * w->cols * es;
         e = launch_gemv_float(base, w->type, 0, x, w->cols, y, w->rows, (uint32_t)batch, (uint32_t)w->rows,
-                              (uint32_t)w->cols, ctx->stream);
+                              (uint32_t)w->cols, ctx->num_cu, ctx->stream);
         return e == hipSuccess ? MMHIP_OK : hip_fail(e, "qmm: launch");
     }
     if (!qmm_fused(w, batch)) {

@@ -621,8 +621,10 @@ hipError_t launch_gemv_segments(const GemvArgs* segs_in, uint32_t n_segs, uint32
 
 hipError_t launch_gemv_float(const void* w, uint32_t type, uint64_t mat_stride, const float* x,
                              uint64_t x_stride, float* y, uint64_t y_stride, uint32_t n_mats,
-                             uint32_t rows, uint32_t cols, hipStream_t s) {
+                             uint32_t rows, uint32_t cols, int num_cu, hipStream_t s) {
     if ((uint64_t)n_mats * rows == 0) return hipSuccess;
+    if (mat_stride == 0 && n_mats > 1 && gemm_strict_fits(n_mats, rows, cols, x_stride, num_cu))
+        return launch_gemm_strict(w, type, x, x_stride, y, y_stride, n_mats, rows, cols, num_cu, s);
     if (mat_stride == 0 && n_mats > 1) {
         // One matrix, several vectors: 16 vectors per workgroup.
         const dim3 grid(rows, (n_mats + 15) / 16);

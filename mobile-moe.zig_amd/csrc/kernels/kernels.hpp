@@ -237,7 +237,13 @@ hipError_t noalloc_scratch(int device, void** out);
 // y_i = W_{first+i} . x_i for i < n_mats.
 hipError_t launch_gemv_float(const void* w, uint32_t ggml_type, uint64_t mat_stride,
                              const float* x, uint64_t x_stride, float* y, uint64_t y_stride,
-                             uint32_t n_mats, uint32_t rows, uint32_t cols, hipStream_t s);
+                             uint32_t n_mats, uint32_t rows, uint32_t cols, int num_cu, hipStream_t s);
+
+// The same for one matrix and n vectors, tiled over rows and vectors
+// (gemm_strict.hip), for the calls gemm_strict_fits accepts.
+bool gemm_strict_fits(uint32_t n, uint32_t rows, uint32_t cols, uint64_t x_stride, int num_cu);
+hipError_t launch_gemm_strict(const void* w, uint32_t ggml_type, const float* x, uint64_t x_stride, float* y,
+                              uint64_t y_stride, uint32_t n, uint32_t rows, uint32_t cols, int num_cu, hipStream_t s);
 
 // Quantised matmul over items of <= 8 activation rows (group.hip).
 // Dense: Y = X . W^T for `batch` rows; out_layout 0: y[b * y_ld + r],

@@ -236,7 +236,8 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
     const bool fused = T == 1 && L->decode_fused;
     if (!fused) {
         TimedLaunch tl(ctx, "moe_router");
-        MOE_TRY(check_hip(launch_gemv_float(L->router->plain, L->router_type, 0, hidden, H, L->scores, E, T, E, H, s),
+        MOE_TRY(check_hip(launch_gemv_float(L->router->plain, L->router_type, 0, hidden, H, L->scores, E, T, E, H,
+                                            ctx->num_cu, s),
                           "moe: router"));
     }
     const bool sep_shared = L->has_shared && !L->shared_merged;
