@@ -323,23 +323,31 @@ int qmm_device(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t mat, const float*
                               (uint32_t)w->cols, ctx->num_cu, ctx->stream);
         return e == hipSuccess ? MMHIP_OK : hip_fail(e, "qmm: launch");
     }
-    if (!qmm_fused(w, batch)) {
+    if (qmm_path(ctx, w, batch) == QmmPath::kTwoLaunch) {
         e = qscratch->ensure(quant_act_bytes(batch, w->geom.cols_pad));
         if (e != hipSuccess) return hip_fail(e, "qmm: scratch");
     }
     return qmm_quantised(ctx, w, mat, x, y, batch, out_layout, qscratch->p, true);
 }
 
-bool qmm_fused(const mmhip_weight* w, uint64_t batch) {
-    // MMHIP_QMM_FUSED=0: the two-launch path (quantize_kernel, then
-    // group_kernel) for every shape.
+QmmPath qmm_path(const mmhip_ctx* ctx, const mmhip_weight* w, uint64_t batch) {
+    // MMHIP_QMM_FUSED=0: never the digit kernel where the tile kernel can run.
     static const bool on = [] {
         const char* e = getenv("MMHIP_QMM_FUSED");
         return !(e && e[0] == '0');
     }();
-    // The fused kernel addresses x (batch rows of cols floats) with 32-bit
-    // byte offsets.
-    return on && qmm_q8_fused_fits(w->geom) && batch * w->cols * 4 < 0x80000000ull;
+    // The digit kernel's many small workgroups end first while they all run
+    // at once, one per CU ([768 x 2048] times 64: 5.9 us against 6.3,
+    // [3840 x 768] times 32: 4.6 against 4.9); past that the tile kernel's
+    // larger tiles do ([768 x 2048] times 256: 8.9 us against 11.2,
+    // [3840 x 768] times 48: 5.8 against 7.5, times 256: 11.3 against 19.8).
+    // Both address x with 32-bit byte offsets.
+    const TileGeom& g = w->geom;
+    if (gemm_tile_fits(g, batch, w->cols)) {
+        const bool small = qmm_q8_fused_workgroups(g, batch) <= (uint64_t)ctx->num_cu;
+        return on && qmm_q8_fused_fits(g) && small ? QmmPath::kFusedQ8 : QmmPath::kTile;
+    }
+    return QmmPath::kTwoLaunch;
 }
 
 int qmm_quantised(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t mat, const float* x, float* y, uint64_t batch,
@@ -347,7 +355,15 @@ int qmm_quantised(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t mat, const flo
     const TileGeom& g = w->geom;
     const uint64_t ld = out_layout == 0 ? w->rows : batch;
     hipError_t e;
-    if (qmm_fused(w, batch)) {
+    const QmmPath path = qmm_path(ctx, w, batch);
+    if (path == QmmPath::kTile) {
+        // One launch reading the f32 activations (qbuf unused).
+        TimedLaunch tl(timed ? ctx : nullptr, "qmm");
+        e = launch_gemm_tile(w->recs, w->dvals, g, mat, false, x, w->cols, (uint32_t)batch, y, out_layout == 0 ? ld : 1,
+                             out_layout == 0 ? 1 : ld, ctx->num_cu, ctx->stream);
+        return e == hipSuccess ? MMHIP_OK : hip_fail(e, "qmm: launch");
+    }
+    if (path == QmmPath::kFusedQ8) {
         // One launch, the activations quantised inside (qbuf unused).
         TimedLaunch tl(timed ? ctx : nullptr, "qmm");
         e = launch_qmm_q8_fused(w->recs, w->dvals, g, mat, x, w->cols, (uint32_t)w->cols, (uint32_t)batch, y, ld,

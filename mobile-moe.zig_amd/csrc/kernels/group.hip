@@ -691,6 +691,11 @@ static uint32_t qmm_q8_slices(const TileGeom& g) {
 
 bool qmm_q8_fused_fits(const TileGeom& g) { return qmm_q8_slices(g) != 0; }
 
+uint64_t qmm_q8_fused_workgroups(const TileGeom& g, uint64_t batch) {
+    const uint32_t ks = qmm_q8_slices(g);
+    return ks ? (g.tiles + 16 / ks - 1) / (16 / ks) * ((batch + kGRows - 1) / kGRows) : 0;
+}
+
 hipError_t launch_qmm_q8_fused(const uint4* recs, const uint16_t* dvals, const TileGeom& g, uint64_t mat,
                                const float* x, uint64_t x_stride, uint32_t cols, uint32_t batch, float* y,
                                uint64_t y_ld, int out_layout, hipStream_t s) {

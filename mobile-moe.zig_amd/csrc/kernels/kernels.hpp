@@ -257,6 +257,7 @@ hipError_t launch_group_dense(const uint4* recs, const uint16_t* dvals, const Ti
 // (K <= 2048 columns). x rows are x_stride floats apart; columns >= cols
 // read as zero.
 bool qmm_q8_fused_fits(const TileGeom& g);
+uint64_t qmm_q8_fused_workgroups(const TileGeom& g, uint64_t batch);  // 0 where it does not fit
 hipError_t launch_qmm_q8_fused(const uint4* recs, const uint16_t* dvals, const TileGeom& g, uint64_t mat,
                                const float* x, uint64_t x_stride, uint32_t cols, uint32_t batch, float* y,
                                uint64_t y_ld, int out_layout, hipStream_t s);
@@ -266,6 +267,23 @@ hipError_t launch_qmm_q8_fused(const uint4* recs, const uint16_t* dvals, const T
 hipError_t launch_group_experts(const uint4* recs, const uint16_t* dvals, const TileGeom& g, const QuantAct& xq,
                                 const uint32_t* a_row, const QmmWork* work, const uint32_t* n_work, uint32_t max_work,
                                 float* y, uint64_t y_ld, int num_cu, hipStream_t s);
+
+// f32 vectors times quantised weights on the bf16 matrix cores
+// (gemm_tile.hip), the vectors read as they are (columns a multiple of 32,
+// x_rows rows x_stride floats apart, below 2 GiB: gemm_tile_fits).
+// y[j * y_slot + r * y_row] = x[j] . W[r]; gate_up: y = silu(x . W_mat[r]) *
+// (x . W_mat+1[r]). Experts: item i < *n_work takes slots [slot, slot +
+// count) (count <= kTileTokens; x row x_row[slot], or the slot itself when
+// x_row is null) and matrix work[i].mat (gate_up: up matrix work[i].pad).
+constexpr uint32_t kTileTokens = 32;
+bool gemm_tile_fits(const TileGeom& g, uint64_t x_rows, uint64_t x_stride);
+hipError_t launch_gemm_tile(const uint4* recs, const uint16_t* dvals, const TileGeom& g, uint64_t mat, bool gate_up,
+                            const float* x, uint64_t x_stride, uint32_t batch, float* y, uint64_t y_slot,
+                            uint64_t y_row, int num_cu, hipStream_t s);
+hipError_t launch_gemm_tile_experts(const uint4* recs, const uint16_t* dvals, const TileGeom& g, bool gate_up,
+                                    const float* x, uint64_t x_stride, uint64_t x_rows, const uint32_t* x_row,
+                                    const QmmWork* work, const uint32_t* n_work, uint32_t max_work, float* y,
+                                    uint64_t y_slot, hipStream_t s);
 
 // Quantises silu(g) * u per row (rows r < *n_rows, or n_rows_max when
 // n_rows is null): g = src + r * src_stride, u = g + u_off.
