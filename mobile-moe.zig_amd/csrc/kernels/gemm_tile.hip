@@ -1,5 +1,7 @@
 // Quantised weights times several f32 vectors on gfx950's bf16 matrix cores:
-// prompt prefill (qmm.matMulQ8_0's role, qmm.zig:58-138).
+// prompt prefill (qmm.matMulQ8_0's role, qmm.zig:58-138) and the MoE experts
+// of a batch grouped by expert (moeFFN over forwardBatch's tokens,
+// inference.zig:346-351, 886-1188; gate, up and silu(gate) * up in one launch).
 //
 // The integer weights of both formats (int8 codes; grid magnitudes with their
 // signs) are exact in bf16, and a vector element is two bf16 numbers
@@ -17,7 +19,8 @@
 // times 32: 16.7 us against 12.9), splits them and turns them into operands
 // through LDS of its own, and reads weights as the record layout has them.
 // Four projections of a layer (768 / 3840 / 576 / 2048 rows): Q8_0 at 256
-// tokens 83.7 -> 45.6 us, IQ2_XXS at 77 tokens 54.1 -> 34.6 us.
+// tokens 83.7 -> 45.6 us, IQ2_XXS at 77 tokens 54.1 -> 34.6 us. Q8_0 MoE layer
+// (64 experts of 1536, hidden 2048) at 256 tokens 405 -> 205 us.
 #include "device_common.hpp"
 #include "gemm_tile_ops.hpp"
 #include "kernels.hpp"
@@ -27,9 +30,10 @@ namespace mmhip {
 namespace {
 
 // Waves of a workgroup split the columns: wave v takes the v-th share of the
-// tile's column steps and the shares are added at the end.
+// tile's column turns and the shares are added at the end. Four waves per SIMD
+// (128 registers) where a wave holds 16 rows of x; 32 need 192 and more.
 template <int FMT, int MT, int NJ, int KS, bool GU>
-__global__ __launch_bounds__(KS * 64, 2) void gemm_tile_kernel(GemmTileArgs a) {
+__global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(GemmTileArgs a) {
     // The waves' activation copies and the IQ2_XXS tables, then the sums.
     constexpr uint32_t kSlot = MT * NJ * 4 * 64;  // floats of a wave's sums
     constexpr uint32_t kRed = KS / 2 * kSlot * 4, kX = tile_lds_bytes<MT>();
@@ -160,8 +164,10 @@ struct TileShape {
 template <int FMT, bool GU>
 const void* tile_fn(const TileShape& t) {
     if (t.mt == 1)
-        return t.nj == 2 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 2, 8, GU>)
-                         : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 4, 8, GU>);
+        return t.ks == 8 ? (t.nj == 2 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 2, 8, GU>)
+                                      : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 4, 8, GU>))
+                         : (t.nj == 2 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 2, 4, GU>)
+                                      : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 4, 4, GU>));
     return t.ks == 8 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 2, 4, 8, GU>)
                      : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 2, 4, 4, GU>);
 }
@@ -244,7 +250,7 @@ hipError_t launch_gemm_tile(const uint4* recs, const uint16_t* dvals, const Tile
 
 hipError_t launch_gemm_tile_experts(const uint4* recs, const uint16_t* dvals, const TileGeom& g, bool gate_up,
                                     const float* x, uint64_t x_stride, uint64_t x_rows, const uint32_t* x_row,
-                                    const QmmWork* work, const uint32_t* n_work, uint32_t max_work, float* y,
+                                    const QmmWork* work, const uint32_t* n_work, uint32_t max_work, uint32_t n_tokens, float* y,
                                     uint64_t y_slot, hipStream_t s) {
     if (!gemm_tile_fits(g, x_rows, x_stride)) return hipErrorInvalidValue;
     GemmTileArgs a = base(recs, dvals, g, x, x_stride, x_rows, y);
@@ -253,7 +259,13 @@ hipError_t launch_gemm_tile_experts(const uint4* recs, const uint16_t* dvals, co
     a.n_work = n_work;
     a.y_slot = y_slot;
     a.y_row = 1;
-    return launch(a, g.fmt, gate_up, TileShape{2, 4, 4}, max_work, s);
+    // Items of 16 rows and four waves: the many short workgroups need the CU's
+    // other workgroups to cover their start and end (four a CU; 32-row items,
+    // which leave room for two, took 219 us for the layer below, and these
+    // 205). A call of few tokens has few items: half tiles give it twice the
+    // workgroups (2 tokens 34.8 us against 36.6, 16 tokens 53.9 against 57.8;
+    // 64 tokens 104.9 against 93.4).
+    return launch(a, g.fmt, gate_up, TileShape{1, n_tokens <= 16 ? 2 : 4, 4}, max_work, s);
 }
 
 }  // namespace mmhip

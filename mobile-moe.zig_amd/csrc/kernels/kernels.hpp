@@ -62,6 +62,8 @@ struct RouteArgs {
     QmmWork* work_dn;
     uint32_t* n_work;           // [2]: active items of work_gu, work_dn
     uint32_t inter;             // routed expert width (up column offset)
+    uint32_t item_rows = kQmmTokens;  // n_tokens > 1: most rows of an item
+    uint32_t paired = 0;        // 1: work_gu holds one item per gate and up (mat gate, pad the up matrix)
     // Optional, n_tokens > 1: the hidden states' wide quantisation (one
     // scale per 256 columns) for the grouped gate/up, done by extra
     // workgroups of the routing launch (it does not depend on the routing).
@@ -275,14 +277,14 @@ hipError_t launch_group_experts(const uint4* recs, const uint16_t* dvals, const 
 // (x . W_mat+1[r]). Experts: item i < *n_work takes slots [slot, slot +
 // count) (count <= kTileTokens; x row x_row[slot], or the slot itself when
 // x_row is null) and matrix work[i].mat (gate_up: up matrix work[i].pad).
-constexpr uint32_t kTileTokens = 32;
+constexpr uint32_t kTileTokens = 16;
 bool gemm_tile_fits(const TileGeom& g, uint64_t x_rows, uint64_t x_stride);
 hipError_t launch_gemm_tile(const uint4* recs, const uint16_t* dvals, const TileGeom& g, uint64_t mat, bool gate_up,
                             const float* x, uint64_t x_stride, uint32_t batch, float* y, uint64_t y_slot,
                             uint64_t y_row, int num_cu, hipStream_t s);
 hipError_t launch_gemm_tile_experts(const uint4* recs, const uint16_t* dvals, const TileGeom& g, bool gate_up,
                                     const float* x, uint64_t x_stride, uint64_t x_rows, const uint32_t* x_row,
-                                    const QmmWork* work, const uint32_t* n_work, uint32_t max_work, float* y,
+                                    const QmmWork* work, const uint32_t* n_work, uint32_t max_work, uint32_t n_tokens, float* y,
                                     uint64_t y_slot, hipStream_t s);
 
 // Quantises silu(g) * u per row (rows r < *n_rows, or n_rows_max when
@@ -304,7 +306,7 @@ hipError_t launch_quantize_silu(const float* src, uint64_t src_stride, uint64_t 
 
 hipError_t launch_route(const RouteArgs& a, hipStream_t s);
 // Upper bound of the grouped items per list for T tokens and E experts.
-uint32_t route_max_work(uint32_t n_tokens, uint32_t n_experts);
+uint32_t route_max_work(uint32_t n_tokens, uint32_t n_experts, uint32_t item_rows);
 
 // out[t] = sum over the token's routed slots, in route order, of w * eo[slot]
 // (products and sums rounded separately), + eo[shared slot], + bias when

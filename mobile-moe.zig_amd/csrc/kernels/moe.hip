@@ -128,7 +128,7 @@ __device__ void route_body(const RouteArgs& a, RouteLds& L) {
         for (uint32_t base = 0; base < E; base += 64) {
             const uint32_t e = base + lane;
             const uint32_t c = e < E ? s_cnt[e] : 0u;
-            const uint32_t ch = (c + kQmmTokens - 1) / kQmmTokens;
+            const uint32_t ch = (c + a.item_rows - 1) / a.item_rows;
             uint32_t inc = c, inc_ch = ch;
 #pragma unroll
             for (int off = 1; off < 64; off <<= 1) {
@@ -157,28 +157,31 @@ __device__ void route_body(const RouteArgs& a, RouteLds& L) {
             a.slot_tok[slot] = t;
         }
     }
-    // Work items: chunk c of expert e is item s_choff[e] + c (gate and up
-    // interleaved in the gate/up list); the shared expert's chunks follow.
+    // Work items: chunk c of expert e is item s_choff[e] + c; the shared
+    // expert's chunks follow.
+    auto put = [&](uint32_t q, uint32_t gate, uint32_t up, uint32_t down, uint32_t slot, uint32_t m) {
+        if (a.paired) {
+            a.work_gu[q] = QmmWork{gate, slot, m, up};
+        } else {
+            a.work_gu[2 * q] = QmmWork{gate, slot, m, 0};
+            a.work_gu[2 * q + 1] = QmmWork{up, slot, m, a.inter};
+        }
+        a.work_dn[q] = QmmWork{down, slot, m, 0};
+    };
     for (uint32_t e = tid; e < E; e += kRouteThreads) {
         const uint32_t c = s_cnt[e], off = s_off[e], ch0 = s_choff[e];
-        for (uint32_t c0 = 0, q = ch0; c0 < c; c0 += kQmmTokens, ++q) {
-            const uint32_t m = min(kQmmTokens, c - c0);
-            a.work_gu[2 * q] = QmmWork{e, off + c0, m, 0};
-            a.work_gu[2 * q + 1] = QmmWork{E + e, off + c0, m, a.inter};
-            a.work_dn[q] = QmmWork{e, off + c0, m, 0};
-        }
+        for (uint32_t c0 = 0, q = ch0; c0 < c; c0 += a.item_rows, ++q)
+            put(q, e, E + e, e, off + c0, min(a.item_rows, c - c0));
     }
     const uint32_t nch = L.nchunks;
     const bool sh = a.shared && a.shared_merged;
-    const uint32_t sh_chunks = sh ? (T + kQmmTokens - 1) / kQmmTokens : 0;
+    const uint32_t sh_chunks = sh ? (T + a.item_rows - 1) / a.item_rows : 0;
     for (uint32_t c = tid; c < sh_chunks; c += kRouteThreads) {
-        const uint32_t c0 = c * kQmmTokens, m = min(kQmmTokens, T - c0), q = nch + c;
-        a.work_gu[2 * q] = QmmWork{2 * E, 4 * T + c0, m, 0};
-        a.work_gu[2 * q + 1] = QmmWork{2 * E + 1, 4 * T + c0, m, a.inter};
-        a.work_dn[q] = QmmWork{E, 4 * T + c0, m, 0};
+        const uint32_t c0 = c * a.item_rows;
+        put(nch + c, 2 * E, 2 * E + 1, E, 4 * T + c0, min(a.item_rows, T - c0));
     }
     if (tid == 0) {
-        a.n_work[0] = 2 * (nch + sh_chunks);
+        a.n_work[0] = (a.paired ? 1 : 2) * (nch + sh_chunks);
         a.n_work[1] = nch + sh_chunks;
     }
 }
@@ -222,10 +225,10 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
 
 }  // namespace
 
-uint32_t route_max_work(uint32_t n_tokens, uint32_t n_experts) {
+uint32_t route_max_work(uint32_t n_tokens, uint32_t n_experts, uint32_t item_rows) {
     const uint32_t routed = 4 * n_tokens;
-    const uint32_t chunks = (n_experts < routed ? n_experts : routed) + (routed + kQmmTokens - 1) / kQmmTokens +
-                            (n_tokens + kQmmTokens - 1) / kQmmTokens;
+    const uint32_t chunks = (n_experts < routed ? n_experts : routed) + (routed + item_rows - 1) / item_rows +
+                            (n_tokens + item_rows - 1) / item_rows;
     return 2 * chunks;
 }
 

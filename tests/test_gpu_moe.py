@@ -194,6 +194,28 @@ def test_q8_experts(ctx, orc, t):
         gpu.free()
 
 
+@pytest.mark.parametrize("variant", ["merged", "narrower", "other_type", "none"])
+@pytest.mark.parametrize("t,hidden,inter", [(2, 512, 256), (16, 544, 288), (17, 288, 32), (67, 768, 160), (256, 256, 512)])
+def test_q8_expert_groups(ctx, orc, t, hidden, inter, variant):
+    """Grouped Q8_0 experts at ragged widths and at the edges of their 16-row
+    items (five experts share the tokens), with every kind of shared expert."""
+    shared_inter = {"merged": inter, "narrower": 256 if inter > 256 else 32, "other_type": 256, "none": None}[variant]
+    shared_fmt = mm.IQ2_XXS if variant == "other_type" and hidden % 256 == 0 else None
+    rng = np.random.default_rng(370 + t)
+    E = 5
+    router, gate, up, down, shared = _weights(rng, mm.Q8_0, hidden, inter, E, shared_inter=shared_inter,
+                                              shared_fmt=shared_fmt, router_sigma=0.05)
+    gpu, cpu = _layers(ctx, orc, mm.Q8_0, hidden, inter, E, router, gate, up, down, shared,
+                       shared_inter=shared_inter, shared_fmt=shared_fmt)
+    try:
+        h = rng.standard_normal((t, hidden)).astype(np.float32)
+        out_g, ids_g, w_g = gpu.ffn(h)
+        out_c, ids_c, w_c = cpu.ffn(h)
+        _check(orc, router, h, out_g, ids_g, w_g, out_c, ids_c, w_c)
+    finally:
+        gpu.free()
+
+
 @pytest.mark.parametrize("t", [1, 6])
 @pytest.mark.parametrize("variant", ["wider", "other_type", "none"])
 def test_shared_expert_variants(ctx, orc, t, variant):
