@@ -63,6 +63,8 @@ struct RouteArgs {
     uint32_t* n_work;           // [2]: active items of work_gu, work_dn
     uint32_t inter;             // routed expert width (up column offset)
     uint32_t item_rows = kQmmTokens;  // n_tokens > 1: most rows of an item
+    uint64_t* tok = nullptr;    // n_tokens > 1: [n_tokens] routed tokens between workgroups
+    uint32_t* ticket = nullptr; //               workgroups that have routed, 0 between calls
     uint32_t paired = 0;        // 1: work_gu holds one item per gate and up (mat gate, pad the up matrix)
     // Optional, n_tokens > 1: the hidden states' wide quantisation (one
     // scale per 256 columns) for the grouped gate/up, done by extra

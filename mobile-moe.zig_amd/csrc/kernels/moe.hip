@@ -1,17 +1,19 @@
 // MoE routing and combine on gfx950 (moeFFN, inference.zig:886-1010).
 //
-// route_kernel: workgroup 0 routes, four tokens per wave (one per 16-lane
-// row); any further workgroups quantise the hidden states for the grouped
-// gate/up meanwhile (one wave per token and 256-column unit). Each token runs
-// Scheduler.route exactly as the CPU path does (math.topK's size-k min-heap,
-// softmax over the selected logits, throttle scaling, the heavy-throttle
-// top-1 fallback) and counts its experts (ExpertStats.counts). The workgroup
-// then lays out the activation slots of the call and writes the problem
-// lists that the expert kernels read on the device, so no routing result
-// travels back to the host:
-//   n_tokens == 1: GEMV problems in route order (decode);
-//   n_tokens >  1: assignments sorted by expert (tokens in order) and cut
-//                  into QMM work items of <= kQmmTokens rows (prefill).
+// route_kernel: workgroups of 16 tokens route (four tokens per wave, one per
+// 16-lane row); further workgroups quantise the hidden states for the grouped
+// IQ2_XXS gate/up meanwhile (one wave per token and 256-column unit). Each
+// token runs Scheduler.route exactly as the CPU path does (math.topK's size-k
+// min-heap, softmax over the selected logits, throttle scaling, the
+// heavy-throttle top-1 fallback). The routing workgroup that ends last counts
+// the experts (ExpertStats.counts), lays out the activation slots of the call
+// and writes the work items that the expert kernels read on the device, so no
+// routing result travels back to the host: assignments sorted by expert
+// (tokens in order) and cut into items of <= item_rows rows.
+//
+// Bound: a token's selection is ~600 dependent vector instructions, so one
+// workgroup for all tokens was bound by its CU (256 tokens 21.5 us, 64 tokens
+// 7.9); sixteen tokens per CU leave one wave per SIMD.
 // combine_kernel: the weighted sum in route order, the shared expert and the
 // deferral bias, with products and sums rounded separately as on the CPU.
 #include "device_common.hpp"
@@ -22,25 +24,83 @@ namespace mmhip {
 
 namespace {
 
-constexpr int kRouteThreads = 1024;  // 16 waves, 4 tokens each at a time
+constexpr int kRouteThreads = 256;   // 4 waves, 4 tokens each
+constexpr uint32_t kRouteTokens = kRouteThreads / 64 * 4;
 constexpr int kMaxTokens = 256;      // MMHIP_MOE_MAX_TOKENS
 constexpr int kMaxExperts = 256;
 
-// LDS of the routing pass (one workgroup of kRouteThreads threads).
+// LDS of a routing workgroup.
 struct RouteLds {
-    uint32_t ids[kMaxTokens * kMaxK];
-    uint32_t act[kMaxTokens];    // bit i: assignment i of the token is computed
+    uint64_t tok[kMaxTokens];    // routed tokens: ids (a byte each), then act from bit 32
     uint32_t cnt[kMaxExperts];   // assignments per expert
     uint32_t rec[kMaxExperts];   // experts recorded in the statistics this call
     uint32_t off[kMaxExperts];   // first slot of each expert
     uint32_t choff[kMaxExperts]; // first work item (chunk) of each expert
     uint32_t rank[kMaxTokens * kMaxK];
-    uint32_t nchunks;
+    uint32_t nchunks, last;
 };
 
-__device__ void route_body(const RouteArgs& a, RouteLds& L) {
-    uint32_t* const s_ids = L.ids;
-    uint32_t* const s_act = L.act;
+// Routes this workgroup's tokens; true in the workgroup that ends last, with
+// every token's word in L.tok.
+__device__ bool route_tokens(const RouteArgs& a, RouteLds& L) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t T = a.n_tokens, E = a.n_experts, k = a.k;
+    const uint32_t n_wg = (T + kRouteTokens - 1) / kRouteTokens;
+    const uint32_t t = blockIdx.x * kRouteTokens + (tid >> 6) * 4 + (lane >> 4);
+    const bool mine = (lane & 15) == 0 && t < T;
+    uint32_t ids[kMaxK], act, deferred;
+    float ts[kMaxK];
+    if (E <= 64)
+        route_select_row16<4>(a, t, ids, ts);
+    else
+        route_select_row16<16>(a, t, ids, ts);
+    route_active(a, act, deferred);
+    // The row's first lane writes the token's results.
+    if (mine) {
+        uint32_t packed = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kMaxK; ++i) packed |= (ids[i] & 0xFFu) << (8 * i);
+        const uint64_t word = (uint64_t)act << 32 | packed;
+        if (n_wg > 1)
+            __hip_atomic_store(a.tok + t, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+            L.tok[t] = word;
+    }
+    if (n_wg > 1) {
+        // The ticket once the words' device-scope stores are performed
+        // (stores count in vmcnt on gfx950).
+        vm_wait_all();
+        lds_barrier();
+        if (tid == 0) {
+            const uint32_t ended = __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            L.last = ended == n_wg - 1;
+            if (L.last) __hip_atomic_store(a.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    // The weights while the ticket is on its way.
+    const TokenRoute tr = finish_route(a, ids, ts);
+    if (mine) {
+        // RouteResult as moeFFN sees it (after the fallback).
+#pragma unroll
+        for (uint32_t i = 0; i < kMaxK; ++i) {
+            if (a.route_ids) a.route_ids[t * kMaxK + i] = i < k ? tr.ids[i] : 0xFFFFFFFFu;
+            if (a.route_w) a.route_w[t * kMaxK + i] = i < k ? tr.w[i] : 0.0f;
+            a.assign_w[t * kMaxK + i] = ((tr.act >> i) & 1u) ? tr.w[i] : 0.0f;
+        }
+        a.deferred[t] = tr.deferred;
+        a.shared_slot[t] = a.shared ? (int32_t)(4 * T + t) : -1;
+        a.slot_tok[4 * T + t] = t;
+    }
+    if (n_wg > 1) {
+        lds_barrier();
+        if (!L.last) return false;
+        for (uint32_t p = tid; p < T; p += kRouteThreads)
+            L.tok[p] = __hip_atomic_load(a.tok + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return true;
+}
+
+__device__ void route_layout(const RouteArgs& a, RouteLds& L) {
     uint32_t* const s_cnt = L.cnt;
     uint32_t* const s_rec = L.rec;
     uint32_t* const s_off = L.off;
@@ -49,6 +109,8 @@ __device__ void route_body(const RouteArgs& a, RouteLds& L) {
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t T = a.n_tokens, E = a.n_experts, k = a.k;
+    auto id_of = [&](uint32_t t, uint32_t i) { return (uint32_t)(L.tok[t] >> (8 * i)) & 0xFFu; };
+    auto active = [&](uint32_t t, uint32_t i) { return i < k && ((L.tok[t] >> (32 + i)) & 1u); };
     for (uint32_t e = tid; e < E; e += kRouteThreads) {
         s_cnt[e] = 0;
         s_rec[e] = 0;
@@ -58,70 +120,18 @@ __device__ void route_body(const RouteArgs& a, RouteLds& L) {
     // wave's outstanding global stores and statistics atomics (~1 us each).
     lds_barrier();
 
-    // Four tokens per wave, one per 16-lane row (route_row16); the row's
-    // first lane writes the token's results.
-    for (uint32_t t0 = 4 * wave; t0 < T; t0 += 4 * (kRouteThreads / 64)) {
-        const uint32_t t = t0 + (lane >> 4);
-        const TokenRoute tr = E <= 64 ? route_row16<4>(a, t) : route_row16<16>(a, t);
-        if ((lane & 15) == 0 && t < T) {
-            const uint32_t act = tr.act;
-#pragma unroll
-            for (uint32_t i = 0; i < kMaxK; ++i)
-                if (i < k) atomicAdd(&s_rec[tr.ids[i]], 1u);  // stats.record (220-222)
-            // RouteResult as moeFFN sees it (after the fallback).
-#pragma unroll
-            for (uint32_t i = 0; i < kMaxK; ++i) {
-                if (a.route_ids) a.route_ids[t * kMaxK + i] = i < k ? tr.ids[i] : 0xFFFFFFFFu;
-                if (a.route_w) a.route_w[t * kMaxK + i] = i < k ? tr.w[i] : 0.0f;
-                s_ids[t * kMaxK + i] = tr.ids[i];
-                a.assign_w[t * kMaxK + i] = ((act >> i) & 1u) ? tr.w[i] : 0.0f;
-                a.assign_slot[t * kMaxK + i] = -1;
-            }
-            s_act[t] = act;
-            a.deferred[t] = tr.deferred;
-            a.shared_slot[t] = a.shared ? (int32_t)(4 * T + t) : -1;
-            a.slot_tok[4 * T + t] = t;
-        }
-    }
-    lds_barrier();
-    // Statistics: one device atomic per recorded expert.
-    for (uint32_t e = tid; e < E; e += kRouteThreads)
-        if (s_rec[e]) atomicAdd(a.counts + e, (unsigned long long)s_rec[e]);
-
-    if (T == 1) {
-        // Decode: slots in route order; GEMV problem lists.
-        if (tid == 0) {
-            uint32_t s = 0;
-            for (uint32_t i = 0; i < k; ++i) {
-                if (!((s_act[0] >> i) & 1u)) continue;
-                const uint32_t e = s_ids[i];
-                a.assign_slot[i] = (int32_t)s;
-                a.slot_tok[s] = 0;
-                a.gemv_gu[2 * s] = make_uint4(e, 0, 2 * s, 0);
-                a.gemv_gu[2 * s + 1] = make_uint4(E + e, 0, 2 * s + 1, 0);
-                a.gemv_dn[s] = make_uint4(e, s, s, 0);
-                ++s;
-            }
-            uint32_t n_gu = 2 * s, n_dn = s;
-            if (a.shared && a.shared_merged) {
-                a.gemv_gu[n_gu++] = make_uint4(2 * E, 0, 8, 0);
-                a.gemv_gu[n_gu++] = make_uint4(2 * E + 1, 0, 9, 0);
-                a.gemv_dn[n_dn++] = make_uint4(E, 4, 4, 0);
-            }
-            a.n_gemv[0] = n_gu;
-            a.n_gemv[1] = n_dn;
-        }
-        return;
-    }
-
     // Prefill: assignments grouped by expert. An assignment's rank inside its
     // expert group comes from an LDS counter; rows of a group are independent,
     // so the order inside a group does not change any result.
     for (uint32_t p = tid; p < T * kMaxK; p += kRouteThreads) {
         const uint32_t t = p / kMaxK, i = p % kMaxK;
-        if (i < k && ((s_act[t] >> i) & 1u)) s_rank[p] = atomicAdd(&s_cnt[s_ids[p]], 1u);
+        if (i < k) atomicAdd(&s_rec[id_of(t, i)], 1u);  // stats.record (220-222)
+        if (active(t, i)) s_rank[p] = atomicAdd(&s_cnt[id_of(t, i)], 1u);
     }
     lds_barrier();
+    // Statistics: one device atomic per recorded expert.
+    for (uint32_t e = tid; e < E; e += kRouteThreads)
+        if (s_rec[e]) atomicAdd(a.counts + e, (unsigned long long)s_rec[e]);
     if (wave == 0) {
         // Exclusive scans over experts: slot offsets and chunk (work item) offsets.
         uint32_t carry = 0, carry_ch = 0;
@@ -151,11 +161,12 @@ __device__ void route_body(const RouteArgs& a, RouteLds& L) {
     lds_barrier();
     for (uint32_t p = tid; p < T * kMaxK; p += kRouteThreads) {
         const uint32_t t = p / kMaxK, i = p % kMaxK;
-        if (i < k && ((s_act[t] >> i) & 1u)) {
-            const uint32_t slot = s_off[s_ids[p]] + s_rank[p];
-            a.assign_slot[p] = (int32_t)slot;
+        int32_t slot = -1;
+        if (active(t, i)) {
+            slot = (int32_t)(s_off[id_of(t, i)] + s_rank[p]);
             a.slot_tok[slot] = t;
         }
+        a.assign_slot[p] = slot;
     }
     // Work items: chunk c of expert e is item s_choff[e] + c; the shared
     // expert's chunks follow.
@@ -188,17 +199,17 @@ __device__ void route_body(const RouteArgs& a, RouteLds& L) {
 
 __global__ __launch_bounds__(kRouteThreads) void route_kernel(RouteArgs a) {
     __shared__ RouteLds L;
-    if (blockIdx.x > 0) {
+    const uint32_t n_wg = (a.n_tokens + kRouteTokens - 1) / kRouteTokens;
+    if (blockIdx.x >= n_wg) {
         // Hidden-state quantisation: one wave per (token, 256-column unit).
-        const uint64_t unit = (uint64_t)(blockIdx.x - 1) * (kRouteThreads / 64) + (threadIdx.x >> 6);
+        const uint64_t unit = (uint64_t)(blockIdx.x - n_wg) * (kRouteThreads / 64) + (threadIdx.x >> 6);
         if (unit < (uint64_t)a.n_tokens * a.q_units)
             quantize_unit_wave<false>(a.qx, a.qx_stride, 0, unit / a.q_units, (uint32_t)(unit % a.q_units), a.q_cols,
                                       a.qa.hi, a.qa.lo, a.qa.scale, a.qa.stride, a.qa.scale_stride);
         return;
     }
-    route_body(a, L);
+    if (route_tokens(a, L)) route_layout(a, L);  // uniform over the workgroup
 }
-
 
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ eo, const int32_t* __restrict__ assign_slot,
                                const float* __restrict__ assign_w, const int32_t* __restrict__ shared_slot,
@@ -233,12 +244,13 @@ uint32_t route_max_work(uint32_t n_tokens, uint32_t n_experts, uint32_t item_row
 }
 
 hipError_t launch_route(const RouteArgs& a, hipStream_t s) {
-    if (a.n_tokens == 0 || a.n_tokens > kMaxTokens || a.n_experts > kMaxExperts || a.k == 0 || a.k > kMaxK ||
+    if (a.n_tokens < 2 || a.n_tokens > kMaxTokens || a.n_experts > kMaxExperts || a.k == 0 || a.k > kMaxK ||
         a.k > a.n_experts)
         return hipErrorInvalidValue;
     const uint64_t q_waves = a.qx ? (uint64_t)a.n_tokens * a.q_units : 0;
     const unsigned q_wgs = (unsigned)((q_waves + kRouteThreads / 64 - 1) / (kRouteThreads / 64));
-    route_kernel<<<1 + q_wgs, kRouteThreads, 0, s>>>(a);
+    const unsigned r_wgs = (a.n_tokens + kRouteTokens - 1) / kRouteTokens;
+    route_kernel<<<r_wgs + q_wgs, kRouteThreads, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -319,7 +319,7 @@ __device__ __forceinline__ int row_max16i(int v) {
 // score of the row equals it as a float; the k picks of clean rounds are
 // distinct and above every other score, which is math.topK's result.
 template <int NC>
-__device__ inline TokenRoute route_row16(const RouteArgs& a, uint32_t t) {
+__device__ inline void route_select_row16(const RouteArgs& a, uint32_t t, uint32_t (&ids)[kMaxK], float (&ts)[kMaxK]) {
     const uint32_t lane = threadIdx.x & 63, p = lane & 15, row = lane >> 4;
     const uint32_t E = a.n_experts, k = a.k;
     const bool live = t < a.n_tokens;
@@ -335,8 +335,11 @@ __device__ inline TokenRoute route_row16(const RouteArgs& a, uint32_t t) {
         bad |= v && sc[c] != sc[c];
         key[c] = v ? order_key(sc[c]) : kKeyNone;
     }
-    uint32_t ids[kMaxK] = {0, 0, 0, 0};
-    float ts[kMaxK] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (uint32_t r = 0; r < kMaxK; ++r) {
+        ids[r] = 0;
+        ts[r] = 0.0f;
+    }
 #pragma unroll
     for (uint32_t r = 0; r < kMaxK; ++r) {  // constant r: ids / ts stay in registers
         if (r >= k) break;
@@ -375,7 +378,6 @@ __device__ inline TokenRoute route_row16(const RouteArgs& a, uint32_t t) {
             ts[i] = __shfl(ts[i], (int)(16 * row), 64);
         }
     }
-    return finish_route(a, ids, ts);
 }
 
 __device__ inline TokenRoute route_token(const RouteArgs& a, uint32_t t) {

@@ -61,6 +61,8 @@ struct mmhip_moe_layer {
     int32_t* shared_slot = nullptr;
     uint32_t* deferred = nullptr;
     uint32_t* slot_tok = nullptr;
+    uint64_t* route_tok = nullptr;
+    uint32_t* route_ticket = nullptr;
     uint4* gemv_gu = nullptr;
     uint4* gemv_dn = nullptr;
     uint32_t* n_gemv = nullptr;
@@ -139,6 +141,8 @@ size_t carve(mmhip_moe_layer* L, char* base) {
     L->shared_slot = (int32_t*)take(T * 4);
     L->deferred = (uint32_t*)take(T * 4);
     L->slot_tok = (uint32_t*)take(S * 4);
+    L->route_tok = (uint64_t*)take(T * 8);
+    L->route_ticket = (uint32_t*)take(4);
     L->gemv_gu = (uint4*)take(10 * 16);
     L->gemv_dn = (uint4*)take(5 * 16);
     L->n_gemv = (uint32_t*)take(2 * 4);
@@ -240,6 +244,8 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
     r.shared_slot = L->shared_slot;
     r.deferred = L->deferred;
     r.slot_tok = L->slot_tok;
+    r.tok = L->route_tok;
+    r.ticket = L->route_ticket;
     r.gemv_gu = L->gemv_gu;
     r.gemv_dn = L->gemv_dn;
     r.n_gemv = L->n_gemv;
