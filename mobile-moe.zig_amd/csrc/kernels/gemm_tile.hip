@@ -32,7 +32,8 @@ namespace {
 // Waves of a workgroup split the columns: wave v takes the v-th share of the
 // tile's column turns and the shares are added at the end. Four waves per SIMD
 // (128 registers) where a wave holds 16 rows of x; 32 need 192 and more.
-template <int FMT, int MT, int NJ, int KS, bool GU>
+// Experts: the items of a.work over packed rows; gate/up leaves packed rows too.
+template <int FMT, int MT, int NJ, int KS, bool GU, bool EXPERTS>
 __global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(GemmTileArgs a) {
     // The waves' activation copies and the IQ2_XXS tables, then the sums.
     constexpr uint32_t kSlot = MT * NJ * 4 * 64;  // floats of a wave's sums
@@ -46,7 +47,7 @@ __global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(Gem
     // of its items.
     const uint32_t xcd = blockIdx.x & 7, r8 = blockIdx.x >> 3;
     uint32_t item, tg;
-    if (a.work) {  // item-major: the items of one expert follow each other
+    if (EXPERTS) {  // item-major: the items of one expert follow each other
         item = r8 / a.groups8;
         tg = (r8 % a.groups8) * 8 + xcd;
         if (item >= *a.n_work) return;
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(Gem
 
     uint32_t first, count;
     uint64_t mat, mat2;
-    if (a.work) {
+    if (EXPERTS) {
         const QmmWork w = a.work[item];
         first = w.slot;
         count = w.count;
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(Gem
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    TileStream<FMT, MT, NJ, GU> st;
+    TileStream<FMT, MT, NJ, GU, EXPERTS> st;
     st.init(a, first, count, mat, mat2, tg, lane);
     uint8_t* const xs = lds + wave * kX;
     const uint32_t s0 = a.turns * wave / KS, s1 = a.turns * (wave + 1) / KS;
@@ -150,7 +151,12 @@ __global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(Gem
             // expertFFN's activation (inference.zig:1179-1180).
             if (GU) v = silu(v) * sum(m, j + kOut, r);
             const uint32_t t = m * 16 + 4 * g + r;
-            if (t < count && row < a.rows) a.y[(uint64_t)(first + t) * a.y_slot + (uint64_t)row * a.y_row] = v;
+            if (t >= count || row >= a.rows) continue;
+            float* const out = a.y + (uint64_t)(first + t) * a.y_slot;
+            if (GU && EXPERTS)
+                pack_row(out, a.rows, row, v);
+            else
+                out[(uint64_t)row * a.y_row] = v;
         }
     }
 }
@@ -162,14 +168,22 @@ struct TileShape {
 };
 
 template <int FMT, bool GU>
-const void* tile_fn(const TileShape& t) {
+const void* dense_fn(const TileShape& t) {
     if (t.mt == 1)
-        return t.ks == 8 ? (t.nj == 2 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 2, 8, GU>)
-                                      : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 4, 8, GU>))
-                         : (t.nj == 2 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 2, 4, GU>)
-                                      : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 4, 4, GU>));
-    return t.ks == 8 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 2, 4, 8, GU>)
-                     : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 2, 4, 4, GU>);
+        return t.nj == 2 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 2, 8, GU, false>)
+                         : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 4, 8, GU, false>);
+    return t.ks == 8 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 2, 4, 8, GU, false>)
+                     : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 2, 4, 4, GU, false>);
+}
+template <int FMT, bool GU>
+const void* experts_fn(const TileShape& t) {
+    return t.nj == 2 ? reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 2, 4, GU, true>)
+                     : reinterpret_cast<const void*>(&gemm_tile_kernel<FMT, 1, 4, 4, GU, true>);
+}
+template <bool GU>
+const void* tile_fn(uint32_t fmt, bool experts, const TileShape& t) {
+    if (fmt == kFmtIq2) return experts ? experts_fn<kFmtIq2, GU>(t) : dense_fn<kFmtIq2, GU>(t);
+    return experts ? experts_fn<kFmtQ8, GU>(t) : dense_fn<kFmtQ8, GU>(t);
 }
 
 uint32_t groups_of(uint32_t tiles, bool gu, const TileShape& t) {
@@ -202,8 +216,8 @@ hipError_t launch(GemmTileArgs& a, uint32_t fmt, bool gu, const TileShape& t, ui
     a.n_items = items;
     const uint64_t blocks = (uint64_t)a.groups8 * items * 8;
     if (blocks > 0x7FFFFFFFu) return hipErrorInvalidValue;
-    const void* fn = fmt == kFmtIq2 ? (gu ? tile_fn<kFmtIq2, true>(t) : tile_fn<kFmtIq2, false>(t))
-                                    : (gu ? tile_fn<kFmtQ8, true>(t) : tile_fn<kFmtQ8, false>(t));
+    const bool experts = a.work != nullptr;
+    const void* fn = gu ? tile_fn<true>(fmt, experts, t) : tile_fn<false>(fmt, experts, t);
     void* args[] = {&a};
     return hipLaunchKernel(fn, dim3((unsigned)blocks), dim3(t.ks * 64), args, 0, s);
 }

@@ -60,6 +60,17 @@ __device__ __forceinline__ void split_bf16(const uint4& q, uint2& hi, uint2& lo)
     lo = make_uint2(l[0], l[1]);
 }
 
+// A packed row of `cols` values takes the bytes of its f32 row: cols bf16 of
+// the first parts, then cols bf16 of the second.
+__device__ __forceinline__ void pack_row(float* row, uint32_t cols, uint32_t col, float v) {
+    const f32x2 p = {v * kActScale, 0.0f};
+    const uint16_t h = (uint16_t)__builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2));
+    const f32x2 d = {p[0] - __uint_as_float((uint32_t)h << 16), 0.0f};
+    uint16_t* r16 = reinterpret_cast<uint16_t*>(row);
+    r16[col] = h;
+    r16[cols + col] = (uint16_t)__builtin_bit_cast(uint32_t, __builtin_convertvector(d, bf16x2));
+}
+
 // Eight int8 weights as bf16 (exact: at most eight significant bits). The
 // conversions leave zeros below the upper half, which v_perm_b32 picks.
 __device__ __forceinline__ bf16x8 q8_bop(uint32_t w0, uint32_t w1) {
@@ -143,11 +154,13 @@ __device__ __forceinline__ void broadcast_rows4(float v, float (&out)[4]) {
 
 // NJ 16-row weight tiles per wave; GU: the first half gate tiles, the others
 // the up tiles of the same rows.
-template <int FMT, int MT, int NJ, bool GU>
+// PACKED: x rows hold two bf16 planes (pack_row) instead of f32 values.
+template <int FMT, int MT, int NJ, bool GU, bool PACKED>
 struct TileStream {
     static constexpr uint32_t kRowTiles = GU ? NJ / 2 : NJ;
-    // Loads in flight: both halves' activations (lane l: rows 4 i + l / 16,
-    // columns 4 (l % 16) .. + 3) and weights of a turn, and the scales of the
+    // Loads in flight: both halves' activations (lane l: f32 rows 4 i + l / 16,
+    // columns 4 (l % 16) .. + 3; packed plane i % 2 of rows 8 (i / 2) + l / 8,
+    // columns 8 (l % 8) .. + 7) and weights of a turn, and the scales of the
     // wave's 64 weight rows (lane l: row l).
     uint4 x[2][MT * 4];
     uint4 q8[2][FMT == kFmtQ8 ? NJ : 1];
@@ -156,7 +169,9 @@ struct TileStream {
 
     BufRsrc x_r, rec_r, rec2_r;
     const uint16_t* d_lane;
-    uint32_t x_voff[MT * 4];
+    static constexpr uint32_t kRowLanes = PACKED ? 8 : 16;
+    static constexpr int kXRows = PACKED ? MT * 2 : MT * 4;
+    uint32_t x_voff[kXRows];
     uint32_t rec_voff, col_lane, tile0, tiles, units, cols;
 
     __device__ __forceinline__ void init(const GemmTileArgs& a, uint32_t first, uint32_t count, uint64_t mat,
@@ -166,15 +181,15 @@ struct TileStream {
         if (GU) rec2_r = make_rsrc(a.recs + mat2 * a.rec_stride, (uint32_t)(a.rec_stride * 16));
         // Rows past the item read zeros (no memory access).
 #pragma unroll
-        for (int i = 0; i < MT * 4; ++i) {
-            const uint32_t j = 4 * i + (lane >> 4);
+        for (int i = 0; i < kXRows; ++i) {
+            const uint32_t j = 64 / kRowLanes * i + lane / kRowLanes;
             const bool ok = j < count;
             uint32_t row = first + (ok ? j : 0);
             if (a.x_row) row = a.x_row[row];
-            x_voff[i] = ok ? row * (a.x_stride * 4) + (lane & 15) * 16 : kBufOob;
+            x_voff[i] = ok ? row * (a.x_stride * 4) + lane % kRowLanes * 16 : kBufOob;
         }
         rec_voff = lane * 16;
-        col_lane = (lane & 15) * 4;
+        col_lane = lane % kRowLanes * (64 / kRowLanes);
         tile0 = tg * kRowTiles;
         tiles = a.tiles;
         units = a.units;
@@ -192,7 +207,12 @@ struct TileStream {
         const uint32_t col = s * kTileTurn + 64 * h;
         const bool in = s < end && col + col_lane < cols;
 #pragma unroll
-        for (int i = 0; i < MT * 4; ++i) x[h][i] = buf_load_b128(x_r, in ? x_voff[i] : kBufOob, col * 4);
+        for (int i = 0; i < MT * 4; ++i) {
+            if constexpr (PACKED)
+                x[h][i] = buf_load_b128(x_r, in ? x_voff[i >> 1] : kBufOob, col * 2 + (i & 1) * (cols * 2));
+            else
+                x[h][i] = buf_load_b128(x_r, in ? x_voff[i] : kBufOob, col * 4);
+        }
     }
     __device__ __forceinline__ void load_w(uint32_t s, uint32_t end, int h) {
 #pragma unroll
@@ -244,6 +264,14 @@ struct TileStream {
 
     // Half h's activations into the wave's LDS copy.
     __device__ __forceinline__ void stage(int h, uint8_t* xs) const {
+        if constexpr (PACKED) {
+            const uint32_t lane = threadIdx.x & 63;
+            uint8_t* dst = xs + (lane & 7) * kRunBytes + (lane >> 3) * 16;
+#pragma unroll
+            for (int i = 0; i < MT * 4; ++i)
+                *reinterpret_cast<uint4*>(dst + ((i >> 2) * 2 + (i & 1)) * kPlaneBytes + ((i >> 1) & 1) * 128) = x[h][i];
+            return;
+        }
         const uint32_t lane = threadIdx.x & 63, cq = lane & 15;
         uint8_t* dst = xs + (cq >> 1) * kRunBytes + (lane >> 4) * 16 + (cq & 1) * 8;
 #pragma unroll

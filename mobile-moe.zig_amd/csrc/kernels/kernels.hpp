@@ -73,6 +73,11 @@ struct RouteArgs {
     uint64_t qx_stride = 0;
     uint32_t q_cols = 0, q_units = 0;  // columns, 256-column units (cols_pad / 256)
     QuantAct qa{};
+    // Optional, n_tokens > 1: the hidden states packed for the bf16 experts,
+    // by the same extra workgroups: [n_tokens][hidden] of px_cols columns.
+    const float* px = nullptr;
+    float* px_out = nullptr;
+    uint32_t px_cols = 0;
 };
 
 struct GemvArgs {
@@ -278,7 +283,9 @@ hipError_t launch_group_experts(const uint4* recs, const uint16_t* dvals, const 
 // y[j * y_slot + r * y_row] = x[j] . W[r]; gate_up: y = silu(x . W_mat[r]) *
 // (x . W_mat+1[r]). Experts: item i < *n_work takes slots [slot, slot +
 // count) (count <= kTileTokens; x row x_row[slot], or the slot itself when
-// x_row is null) and matrix work[i].mat (gate_up: up matrix work[i].pad).
+// x_row is null) and matrix work[i].mat (gate_up: up matrix work[i].pad). Its x
+// rows, and the rows that gate_up writes, are packed: in the bytes of an f32 row
+// of g.cols values, two planes of bf16 (launch_route's px).
 constexpr uint32_t kTileTokens = 16;
 bool gemm_tile_fits(const TileGeom& g, uint64_t x_rows, uint64_t x_stride);
 hipError_t launch_gemm_tile(const uint4* recs, const uint16_t* dvals, const TileGeom& g, uint64_t mat, bool gate_up,

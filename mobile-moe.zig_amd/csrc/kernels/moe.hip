@@ -17,6 +17,7 @@
 // combine_kernel: the weighted sum in route order, the shared expert and the
 // deferral bias, with products and sums rounded separately as on the CPU.
 #include "device_common.hpp"
+#include "gemm_tile_ops.hpp"
 #include "kernels.hpp"
 #include "route_ops.hpp"
 
@@ -201,6 +202,15 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(RouteArgs a) {
     __shared__ RouteLds L;
     const uint32_t n_wg = (a.n_tokens + kRouteTokens - 1) / kRouteTokens;
     if (blockIdx.x >= n_wg) {
+        if (a.px) {
+            // Hidden states as bf16 pairs.
+            const uint64_t i = (uint64_t)(blockIdx.x - n_wg) * kRouteThreads + threadIdx.x;
+            if (i < (uint64_t)a.n_tokens * a.px_cols) {
+                const uint32_t t = (uint32_t)(i / a.px_cols), col = (uint32_t)(i % a.px_cols);
+                pack_row(a.px_out + (uint64_t)t * a.px_cols, a.px_cols, col, a.px[i]);
+            }
+            return;
+        }
         // Hidden-state quantisation: one wave per (token, 256-column unit).
         const uint64_t unit = (uint64_t)(blockIdx.x - n_wg) * (kRouteThreads / 64) + (threadIdx.x >> 6);
         if (unit < (uint64_t)a.n_tokens * a.q_units)
@@ -248,7 +258,8 @@ hipError_t launch_route(const RouteArgs& a, hipStream_t s) {
         a.k > a.n_experts)
         return hipErrorInvalidValue;
     const uint64_t q_waves = a.qx ? (uint64_t)a.n_tokens * a.q_units : 0;
-    const unsigned q_wgs = (unsigned)((q_waves + kRouteThreads / 64 - 1) / (kRouteThreads / 64));
+    const uint64_t p_waves = a.px ? ((uint64_t)a.n_tokens * a.px_cols + 63) / 64 : 0;
+    const unsigned q_wgs = (unsigned)((q_waves + p_waves + kRouteThreads / 64 - 1) / (kRouteThreads / 64));
     const unsigned r_wgs = (a.n_tokens + kRouteTokens - 1) / kRouteTokens;
     route_kernel<<<r_wgs + q_wgs, kRouteThreads, 0, s>>>(a);
     return hipGetLastError();

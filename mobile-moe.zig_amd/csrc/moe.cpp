@@ -77,6 +77,7 @@ struct mmhip_moe_layer {
     void* xq_h = nullptr;    // quantised hidden [T][gu cols_pad]
     void* xq_d = nullptr;    // quantised down input [5 T][dn cols_pad]
     void* xq_sd = nullptr;   // quantised shared down input [T][sh_dn cols_pad]
+    float* xp = nullptr;     // hidden states as bf16 pairs [T][hidden] (Q8_0 experts)
     float* bias = nullptr;   // [hidden]
     // One-launch decode (IQ2_XXS experts): h planes and scales handed from
     // the gate/up workgroups to the down workgroups, and the grid counters.
@@ -157,6 +158,7 @@ size_t carve(mmhip_moe_layer* L, char* base) {
     L->xq_h = take(quant_act_bytes(T, L->gu->geom.cols_pad));
     L->xq_d = take(quant_act_bytes(S, L->dn->geom.cols_pad));
     if (L->has_shared && !L->shared_merged) L->xq_sd = take(quant_act_bytes(T, L->sh_dn->geom.cols_pad));
+    if (L->gu->geom.fmt == kFmtQ8) L->xp = (float*)take(T * H * 4);
     L->bias = (float*)take(H * 4);
     L->dm_hq = (uint8_t*)take(5 * (uint64_t)(I / 32) * 64);
     L->dm_hs = (float*)take(5 * (uint64_t)(I / 32) * 4);
@@ -258,6 +260,9 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
     if (tile) {
         r.item_rows = kTileTokens;
         r.paired = 1;
+        r.px = hidden;
+        r.px_out = L->xp;
+        r.px_cols = H;
     }
     if (!fused) {
         TimedLaunch tl(ctx, "moe_router");
@@ -360,7 +365,7 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
         const uint32_t items = route_max_work(T, E, kTileTokens) / 2;
         {
             TimedLaunch tl(ctx, "moe_gateup");
-            MOE_TRY(check_hip(launch_gemm_tile_experts(L->gu->recs, L->gu->dvals, L->gu->geom, true, hidden, H, T,
+            MOE_TRY(check_hip(launch_gemm_tile_experts(L->gu->recs, L->gu->dvals, L->gu->geom, true, L->xp, H, T,
                                                        L->slot_tok, L->work_gu, L->n_work, items, T, L->y_gu, I, s),
                               "moe: gate/up"));
             if (sep_shared)
