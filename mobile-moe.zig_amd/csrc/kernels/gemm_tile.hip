@@ -20,7 +20,9 @@
 // through LDS of its own, and reads weights as the record layout has them.
 // Four projections of a layer (768 / 3840 / 576 / 2048 rows): Q8_0 at 256
 // tokens 83.7 -> 45.6 us, IQ2_XXS at 77 tokens 54.1 -> 34.6 us. Q8_0 MoE layer
-// (64 experts of 1536, hidden 2048) at 256 tokens 405 -> 205 us.
+// (64 experts of 1536 and a shared one, hidden 2048) at 256 tokens 405 -> 184
+// us, there between the vector instructions (half of the launch) and the L2's
+// traffic (12 TB/s: every item reads its weights again).
 #include "device_common.hpp"
 #include "gemm_tile_ops.hpp"
 #include "kernels.hpp"
@@ -274,12 +276,15 @@ hipError_t launch_gemm_tile_experts(const uint4* recs, const uint16_t* dvals, co
     a.y_slot = y_slot;
     a.y_row = 1;
     // Items of 16 rows and four waves: the many short workgroups need the CU's
-    // other workgroups to cover their start and end (four a CU; 32-row items,
-    // which leave room for two, took 219 us for the layer below, and these
-    // 205). A call of few tokens has few items: half tiles give it twice the
-    // workgroups (2 tokens 34.8 us against 36.6, 16 tokens 53.9 against 57.8;
-    // 64 tokens 104.9 against 93.4).
-    return launch(a, g.fmt, gate_up, TileShape{1, n_tokens <= 16 ? 2 : 4, 4}, max_work, s);
+    // other workgroups to cover their start and end (four a CU; 32-row items
+    // leave room for two and halve the weights' conversions, the same 190 us for
+    // the Q8_0 layer above at 256 tokens and 103 against 91 at 64). A call of few
+    // tokens has few items: half tiles give it twice the workgroups (Q8_0 2
+    // tokens 32.3 us against 34.8, 16 tokens 50.6 against 55.7, 64 tokens 101.5
+    // against 90.6; IQ2_XXS 2 tokens 32.5 against 35.7, 12 tokens 43.7 against
+    // 41.9).
+    const uint32_t few = g.fmt == kFmtIq2 ? 8 : 16;
+    return launch(a, g.fmt, gate_up, TileShape{1, n_tokens <= few ? 2 : 4, 4}, max_work, s);
 }
 
 }  // namespace mmhip

@@ -84,10 +84,13 @@ __device__ __forceinline__ bf16x8 q8_bop(uint32_t w0, uint32_t w1) {
     return __builtin_bit_cast(bf16x8, make_uint4(b[0], b[1], b[2], b[3]));
 }
 
-// IQ2_XXS operand tables (6 KiB): entry idx of the grid as eight bf16
+// IQ2_XXS operand tables (4.5 KiB): entry idx of the grid as eight bf16
 // magnitudes, then for each of 128 sign keys (b012 | P << 3 | hi3 << 4 of the
-// record, device_common.hpp) the eight bf16 sign bits.
-constexpr uint32_t kIq2BfGridWords = 256 * 4, kIq2BfWords = kIq2BfGridWords + 128 * 4;
+// record, device_common.hpp) the eight signs in one word: columns 2 c and
+// 2 c + 1 at bits 15 - c and 31 - c, a shift by c away from their bf16 sign bits
+// (a second 16-byte read per record instead of the shifts: the IQ2_XXS experts
+// below were LDS bound).
+constexpr uint32_t kIq2BfGridWords = 256 * 4, kIq2BfWords = kIq2BfGridWords + 128;
 struct Iq2BfTables {
     uint32_t w[kIq2BfWords];
 };
@@ -104,7 +107,7 @@ constexpr Iq2BfTables make_iq2_bf_tables() {
         const uint32_t b012 = k & 7u, par = (k >> 3) & 1u, h = k >> 4;
         const uint32_t s = b012 | ((par ^ parity3(b012)) << 3) | (h << 4) | ((par ^ parity3(h)) << 7);
         for (uint32_t c = 0; c < 4; ++c)
-            t.w[kIq2BfGridWords + k * 4 + c] = ((s >> (2 * c)) & 1u) << 15 | ((s >> (2 * c + 1)) & 1u) << 31;
+            t.w[kIq2BfGridWords + k] |= ((s >> (2 * c)) & 1u) << (15 - c) | ((s >> (2 * c + 1)) & 1u) << (31 - c);
     }
     return t;
 }
@@ -119,8 +122,10 @@ __device__ __forceinline__ void iq2_bf_table_load(uint32_t* tab) {
 __device__ __forceinline__ bf16x8 iq2_bop_bf16(uint32_t grid_off, uint32_t sign_off, const uint32_t* tab) {
     const char* t = reinterpret_cast<const char*>(tab);
     const uint4 m = *reinterpret_cast<const uint4*>(t + grid_off);
-    const uint4 s = *reinterpret_cast<const uint4*>(t + kIq2BfGridWords * 4 + sign_off);
-    return __builtin_bit_cast(bf16x8, make_uint4(m.x ^ s.x, m.y ^ s.y, m.z ^ s.z, m.w ^ s.w));
+    const uint32_t s = *reinterpret_cast<const uint32_t*>(t + kIq2BfGridWords * 4 + sign_off);
+    constexpr uint32_t k = 0x80008000u;
+    return __builtin_bit_cast(bf16x8, make_uint4(m.x ^ (s & k), m.y ^ ((s << 1) & k), m.z ^ ((s << 2) & k),
+                                                 m.w ^ ((s << 3) & k)));
 }
 
 // A wave's LDS copy of one half turn of its activations, as the products read
@@ -241,19 +246,22 @@ struct TileStream {
     __device__ __forceinline__ void scales(float (&c)[4][4]) const {
         if constexpr (FMT == kFmtIq2) {
             const uint32_t g = (threadIdx.x & 63) >> 4;
-            float d8[4];
+            // (0.5 + ls) / 4 = ls (2 / 8) + 1 / 8 of the row's scale (dequant.zig:336).
+            float d8[4], d2[4];
             broadcast_rows4(f16_scale((uint16_t)d.x) * (0.125f * kActUnscale), d8);
 #pragma unroll
+            for (int j = 0; j < 4; ++j) d2[j] = d8[j] * 2.0f;
+#pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                // Nibble b: sub-block b of the half unit, gathered from the
-                // row's four lane groups.
-                const uint32_t mine = ((iq[j].x >> 30) | ((iq[j].y >> 30) << 2)) << (4 * g);
+                // Byte b: ls of sub-block b of the half unit, gathered from
+                // the row's four lane groups.
+                const uint32_t mine = ((iq[j].x >> 30) | ((iq[j].y >> 30) << 2)) << (8 * g);
                 const auto p = __builtin_amdgcn_permlane16_swap(mine, mine, false, false);
                 const uint32_t pair = p[0] | p[1];
                 const auto q = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
                 const uint32_t ls = q[0] | q[1];
 #pragma unroll
-                for (int b = 0; b < 4; ++b) c[b][j] = (float)(int)(((ls >> (4 * b)) & 15u) * 2 + 1) * d8[j];
+                for (int b = 0; b < 4; ++b) c[b][j] = fmaf((float)((ls >> (8 * b)) & 0xFFu), d2[j], d8[j]);
             }
         } else {
 #pragma unroll
@@ -303,8 +311,8 @@ struct TileStream {
                 bf16x8 w;
                 if constexpr (FMT == kFmtIq2) {
                     const uint32_t dw = h ? iq[j].y : iq[j].x;
-                    w = b ? iq2_bop_bf16((dw >> 18) & 0xFF0u, ((dw >> 14) & 0xF0u) | ((dw << 8) & 0x700u), tab)
-                          : iq2_bop_bf16((dw >> 3) & 0xFF0u, ((dw << 1) & 0xF0u) | ((dw >> 7) & 0x700u), tab);
+                    w = b ? iq2_bop_bf16((dw >> 18) & 0xFF0u, ((dw >> 16) & 0x3Cu) | ((dw << 6) & 0x1C0u), tab)
+                          : iq2_bop_bf16((dw >> 3) & 0xFF0u, ((dw >> 1) & 0x3Cu) | ((dw >> 9) & 0x1C0u), tab);
                 } else {
                     w = b ? q8_bop(q8[h][j].z, q8[h][j].w) : q8_bop(q8[h][j].x, q8[h][j].y);
                 }

@@ -595,6 +595,8 @@ int resident(const void* fn, int wg) {
     return nb;
 }
 
+constexpr uint32_t kLargeTiles = 16;  // item tiles per CU of a 1024-thread launch
+
 hipError_t launch(GroupArgs a, uint32_t fmt, uint32_t items, int num_cu, hipStream_t s) {
     if (items == 0 || a.tiles == 0) return hipSuccess;
     // Workgroup size and step, measured on MI355X at batch 64: IQ2_XXS
@@ -612,9 +614,10 @@ hipError_t launch(GroupArgs a, uint32_t fmt, uint32_t items, int num_cu, hipStre
     static const int wg_env = env_int("MMHIP_GROUP_WG", 0);
     const uint64_t cus = (uint64_t)(num_cu > 0 ? num_cu : 256);
     const uint64_t tiles_all = (uint64_t)items * a.tiles;
+    const bool large = fmt == kFmtIq2 && tiles_all >= cus * kLargeTiles;
     const bool wg_ok = wg_env == 256 || wg_env == 512 || (wg_env == 1024 && fmt == kFmtIq2);
     const int wg = wg_ok                                         ? wg_env
-                   : fmt == kFmtIq2 && tiles_all >= cus * 16 ? 1024
+                   : large ? 1024
                    : fmt == kFmtIq2 && tiles_all >= cus * 8  ? 512
                                                                  : 256;
     const int ups = group_ups(a.units, fmt, wg >= 512 ? 1 : 4);
@@ -739,6 +742,10 @@ hipError_t launch_qmm_q8_fused(const uint4* recs, const uint16_t* dvals, const T
                           reinterpret_cast<const void*>(&qmm_q8_fused_kernel<7>)};
     void* args[] = {&a};
     return hipLaunchKernel(fns[ks], dim3((unsigned)blocks), dim3(tpw * ks * 64), args, 0, s);
+}
+
+bool group_large(const TileGeom& g, uint32_t items, int num_cu) {
+    return g.fmt == kFmtIq2 && (uint64_t)items * g.tiles >= (uint64_t)(num_cu > 0 ? num_cu : 256) * kLargeTiles;
 }
 
 hipError_t launch_group_experts(const uint4* recs, const uint16_t* dvals, const TileGeom& g, const QuantAct& xq,

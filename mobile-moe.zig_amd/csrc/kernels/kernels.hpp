@@ -296,6 +296,9 @@ hipError_t launch_gemm_tile_experts(const uint4* recs, const uint16_t* dvals, co
                                     const QmmWork* work, const uint32_t* n_work, uint32_t max_work, uint32_t n_tokens, float* y,
                                     uint64_t y_slot, hipStream_t s);
 
+// Whether a grouped call of so many items runs in 1024-thread workgroups.
+bool group_large(const TileGeom& g, uint32_t items, int num_cu);
+
 // Quantises silu(g) * u per row (rows r < *n_rows, or n_rows_max when
 // n_rows is null): g = src + r * src_stride, u = g + u_off.
 hipError_t launch_quantize_silu(const float* src, uint64_t src_stride, uint64_t u_off, const uint32_t* n_rows,

@@ -18,11 +18,11 @@
 //                   formed while quantising; with IQ2_XXS
 //                   experts (shared merged) it also does the
 //                   combine in the same launch               "moe_down"
-//   T > 1 (prefill, experts grouped), Q8_0 experts:
+//   T > 1 (prefill, experts grouped), mostly (moe_tile):
 //     gate/up       expert-sorted slots times gate and up, and
 //                   silu(gate) * up                         "moe_gateup"
 //     down                                                  "moe_down"
-//   T > 1, IQ2_XXS experts:
+//   T > 1, other calls of IQ2_XXS experts:
 //     (the routing launch quantises the hidden states)
 //     gate/up       grouped QMM over expert-sorted slots      "moe_gateup"
 //     silu*up       quantised per slot                        "moe_quantize"
@@ -77,7 +77,7 @@ struct mmhip_moe_layer {
     void* xq_h = nullptr;    // quantised hidden [T][gu cols_pad]
     void* xq_d = nullptr;    // quantised down input [5 T][dn cols_pad]
     void* xq_sd = nullptr;   // quantised shared down input [T][sh_dn cols_pad]
-    float* xp = nullptr;     // hidden states as bf16 pairs [T][hidden] (Q8_0 experts)
+    float* xp = nullptr;     // hidden states as bf16 pairs [T][hidden]
     float* bias = nullptr;   // [hidden]
     // One-launch decode (IQ2_XXS experts): h planes and scales handed from
     // the gate/up workgroups to the down workgroups, and the grid counters.
@@ -158,7 +158,7 @@ size_t carve(mmhip_moe_layer* L, char* base) {
     L->xq_h = take(quant_act_bytes(T, L->gu->geom.cols_pad));
     L->xq_d = take(quant_act_bytes(S, L->dn->geom.cols_pad));
     if (L->has_shared && !L->shared_merged) L->xq_sd = take(quant_act_bytes(T, L->sh_dn->geom.cols_pad));
-    if (L->gu->geom.fmt == kFmtQ8) L->xp = (float*)take(T * H * 4);
+    L->xp = (float*)take(T * H * 4);
     L->bias = (float*)take(H * 4);
     L->dm_hq = (uint8_t*)take(5 * (uint64_t)(I / 32) * 64);
     L->dm_hs = (float*)take(5 * (uint64_t)(I / 32) * 4);
@@ -213,12 +213,23 @@ int gemv_launch(mmhip_ctx* ctx, const mmhip_weight* w, const char* family, const
 
 int check_hip(hipError_t e, const char* what) { return e == hipSuccess ? MMHIP_OK : hip_fail(e, what); }
 
-// Whether a call of several tokens runs its experts on the bf16 matrix cores:
-// Q8_0 experts always (2 tokens 47.8 -> 34.8 us, 64 tokens 139 -> 93, 256
-// tokens 405 -> 205), IQ2_XXS keeps the digit kernel (64 tokens 72.5 us against
-// 79.8).
-bool moe_tile(const mmhip_moe_layer* L, uint32_t T) {
-    if (T == 1 || L->gu->geom.fmt != kFmtQ8) return false;
+// Whether a call of several tokens runs its experts on the bf16 matrix cores.
+// Q8_0 experts always (layer of 64 experts of 1536, hidden 2048: 2 tokens 47.0
+// -> 32.3 us, 64 tokens 138 -> 91, 256 tokens 396 -> 188). IQ2_XXS experts keep
+// the digit kernel's 8-row items where a large layer's call has enough of them
+// for its 1024-thread workgroups but few rows each: fewer than the experts, a
+// fifth of an item's cost is then the 16-row tile's empty rows (same layer, 16
+// tokens 46.7 us against 48.0, 48 tokens 62.6 against 66.6, 64 tokens 71.1
+// against 71.4, 256 tokens 158 against 147; 4 tokens, below those workgroups,
+// 49.2 against 39.1; hidden 1024, experts of 512: 64 tokens 39.3 against 31.0). A
+// separate shared expert costs the digit path five launches (92.6 us against
+// 79.6 at 64 tokens).
+bool moe_tile(const mmhip_moe_layer* L, uint32_t T, int num_cu) {
+    if (T == 1) return false;
+    const TileGeom& g = L->gu->geom;
+    if (g.fmt == kFmtIq2 && !L->sh_gu && T < L->n_experts && (uint64_t)L->inter * L->hidden >= (1u << 21) &&
+        group_large(g, route_max_work(T, L->n_experts, kQmmTokens), num_cu))
+        return false;
     if (!gemm_tile_fits(L->gu->geom, T, L->hidden) || !gemm_tile_fits(L->dn->geom, 5 * T, L->inter)) return false;
     return !L->sh_gu || (gemm_tile_fits(L->sh_gu->geom, T, L->hidden) &&
                          gemm_tile_fits(L->sh_dn->geom, T, L->shared_inter));
@@ -256,7 +267,7 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
     r.n_work = L->n_work;
     r.inter = I;
     const bool fused = T == 1 && L->decode_fused;
-    const bool tile = moe_tile(L, T);
+    const bool tile = moe_tile(L, T, ctx->num_cu);
     if (tile) {
         r.item_rows = kTileTokens;
         r.paired = 1;

@@ -216,6 +216,23 @@ def test_q8_expert_groups(ctx, orc, t, hidden, inter, variant):
         gpu.free()
 
 
+@pytest.mark.parametrize("t,n_exp", [(15, 64), (16, 12), (40, 64), (40, 33)])
+def test_iq2_expert_groups_large_layer(ctx, orc, t, n_exp):
+    """A layer large enough that calls of fewer tokens than experts keep the
+    digit kernel's items: both sides of that rule, no shared expert."""
+    hidden, inter = 2048, 1024
+    rng = np.random.default_rng(380 + t + n_exp)
+    w = _weights(rng, mm.IQ2_XXS, hidden, inter, n_exp, router_sigma=0.03)
+    gpu, cpu = _layers(ctx, orc, mm.IQ2_XXS, hidden, inter, n_exp, *w)
+    try:
+        h = rng.standard_normal((t, hidden)).astype(np.float32)
+        out_g, ids_g, w_g = gpu.ffn(h)
+        out_c, ids_c, w_c = cpu.ffn(h)
+        _check(orc, w[0], h, out_g, ids_g, w_g, out_c, ids_c, w_c)
+    finally:
+        gpu.free()
+
+
 @pytest.mark.parametrize("t", [1, 6])
 @pytest.mark.parametrize("variant", ["wider", "other_type", "none"])
 def test_shared_expert_variants(ctx, orc, t, variant):
