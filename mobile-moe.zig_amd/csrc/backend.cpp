@@ -88,6 +88,11 @@ hipError_t HostBuf::ensure(size_t bytes) {
         p = nullptr;
         return e;
     }
+    e = hipHostGetDevicePointer(&dev, p, 0);
+    if (e != hipSuccess) {
+        release();
+        return e;
+    }
     cap = want;
     return hipSuccess;
 }
@@ -95,6 +100,7 @@ hipError_t HostBuf::ensure(size_t bytes) {
 void HostBuf::release() {
     if (p) (void)hipHostFree(p);
     p = nullptr;
+    dev = nullptr;
     cap = 0;
 }
 

@@ -37,6 +37,7 @@ struct DevBuf {
 };
 struct HostBuf {
     void* p = nullptr;
+    void* dev = nullptr;  // the device's address of p
     size_t cap = 0;
     hipError_t ensure(size_t bytes);
     void release();

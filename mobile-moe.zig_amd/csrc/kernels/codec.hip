@@ -442,7 +442,28 @@ __global__ __launch_bounds__(kQ8DqThreads) void dequantize_q8_0_rows_kernel(cons
     }
 }
 
+// Pinned host memory -> device: 16 bytes per thread, the last words singly.
+// Bound: the link.
+__global__ __launch_bounds__(256) void copy_words_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst,
+                                                         uint64_t n) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (4 * i + 4 <= n) {
+        dst[i] = src[i];
+    } else {
+        const uint32_t* s = reinterpret_cast<const uint32_t*>(src);
+        uint32_t* d = reinterpret_cast<uint32_t*>(dst);
+        for (uint64_t w = 4 * i; w < n; ++w) d[w] = s[w];
+    }
+}
+
 }  // namespace
+
+hipError_t launch_copy_words(const uint32_t* src, uint32_t* dst, uint64_t n, hipStream_t s) {
+    if (n == 0) return hipSuccess;
+    copy_words_kernel<<<(unsigned)((n + 1023) / 1024), 256, 0, s>>>(reinterpret_cast<const uint4*>(src),
+                                                                    reinterpret_cast<uint4*>(dst), n);
+    return hipGetLastError();
+}
 
 hipError_t launch_dequant(const void* raw, uint32_t type, uint64_t n, float* out, hipStream_t s) {
     if (n == 0) return hipSuccess;

@@ -130,6 +130,9 @@ struct GemvOneArgs {
     static constexpr const uint32_t* n_active = nullptr;
 };
 
+// Copies n 32-bit words (16-byte aligned ends) from pinned host memory.
+hipError_t launch_copy_words(const uint32_t* src, uint32_t* dst, uint64_t n, hipStream_t s);
+
 // Raw GGUF bytes -> f32, bit-exact (dequant.zig:316-390, 632-659).
 hipError_t launch_dequant(const void* raw, uint32_t ggml_type, uint64_t n, float* out, hipStream_t s);
 

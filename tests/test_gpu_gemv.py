@@ -263,6 +263,19 @@ def test_qmm_reference_kats(ctx, orc):
         assert np.all(np.abs(exp - out[ni]) <= 0.01)
 
 
+@pytest.mark.parametrize("rows,cols,batch", [(3, 2731, 3), (5, 2730, 3), (700, 512, 400), (16, 4099, 32), (16, 4097, 32)])
+def test_seam_batches_by_size(ctx, orc, rows, cols, batch):
+    """Host calls whose vectors or results lie at the sizes where the copies
+    change: every output is the single-vector call's, bit for bit."""
+    rng = np.random.default_rng(rows + cols)
+    raw = rng.standard_normal((rows, cols)).astype(np.float32)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    y = ctx.batch_mat_mul(raw, mm.F32, x, rows, batch, cols)
+    for b in (0, 1, batch // 2, batch - 1):
+        one = ctx.mat_vec_mul(raw, mm.F32, x[b], rows, cols)
+        assert np.array_equal(y[b].view(np.uint32), one.view(np.uint32))
+
+
 def test_seam_is_thread_safe(ctx, orc):
     """The reference re-enters the seam from 4 pool workers at once
     (inference.zig:934-971); 4 threads must get the same answers as 1."""
