@@ -221,27 +221,41 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(RouteArgs a) {
     if (route_tokens(a, L)) route_layout(a, L);  // uniform over the workgroup
 }
 
+// Four columns of one token per thread (VEC: rows of a multiple of four
+// columns, 16-byte aligned), so the token's slots and weights are uniform and
+// its expert rows load together; one column at a time took 2.4 us for one token of
+// 2048 columns against 1.4, 3.9 for 64 against 3.0 and 5.2 for 256 against 4.6.
+template <int VEC>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ eo, const int32_t* __restrict__ assign_slot,
                                const float* __restrict__ assign_w, const int32_t* __restrict__ shared_slot,
                                const uint32_t* __restrict__ deferred, const float* __restrict__ bias,
-                               float* __restrict__ out, uint32_t n_tokens, uint32_t hidden) {
-    // All arguments in one batch of scalar loads (the bounds check below
-    // otherwise waited for its own first: one more round trip).
-    asm volatile("" ::"s"(eo), "s"(assign_slot), "s"(assign_w), "s"(shared_slot), "s"(deferred), "s"(bias), "s"(out),
-                 "s"(n_tokens), "s"(hidden));
-    const uint64_t gid = (uint64_t)blockIdx.x * 256 + threadIdx.x;  // 256 threads (launch_combine)
-    if (gid >= (uint64_t)n_tokens * hidden) return;
-    const uint32_t t = (uint32_t)(gid / hidden), j = (uint32_t)(gid % hidden);
-    float o = 0.0f;
+                               float* __restrict__ out, uint32_t hidden) {
+    typedef float vf __attribute__((ext_vector_type(VEC)));
+    const uint32_t t = blockIdx.y, j = (blockIdx.x * 256 + threadIdx.x) * VEC;
+    if (j >= hidden) return;
+    int32_t s[kMaxK + 1];
+    float w[kMaxK];
 #pragma unroll
     for (int i = 0; i < kMaxK; ++i) {
-        const int32_t s = assign_slot[t * kMaxK + i];
-        if (s >= 0) o = __fadd_rn(o, __fmul_rn(assign_w[t * kMaxK + i], eo[(uint64_t)s * hidden + j]));
+        s[i] = assign_slot[t * kMaxK + i];
+        w[i] = assign_w[t * kMaxK + i];
     }
-    const int32_t sh = shared_slot[t];
-    if (sh >= 0) o = __fadd_rn(o, eo[(uint64_t)sh * hidden + j]);
-    if (bias && deferred[t]) o = __fadd_rn(o, bias[j]);
-    out[gid] = o;
+    s[kMaxK] = shared_slot[t];
+    const bool with_bias = bias && deferred[t];
+    vf v[kMaxK + 1];
+#pragma unroll
+    for (int i = 0; i <= kMaxK; ++i)
+        if (s[i] >= 0) v[i] = *reinterpret_cast<const vf*>(eo + (uint64_t)s[i] * hidden + j);
+    vf o = 0.0f;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+#pragma unroll
+        for (int i = 0; i < kMaxK; ++i)
+            if (s[i] >= 0) o[e] = __fadd_rn(o[e], __fmul_rn(w[i], v[i][e]));
+        if (s[kMaxK] >= 0) o[e] = __fadd_rn(o[e], v[kMaxK][e]);
+        if (with_bias) o[e] = __fadd_rn(o[e], bias[j + e]);
+    }
+    *reinterpret_cast<vf*>(out + (uint64_t)t * hidden + j) = o;
 }
 
 }  // namespace
@@ -268,10 +282,14 @@ hipError_t launch_route(const RouteArgs& a, hipStream_t s) {
 hipError_t launch_combine(const float* eo, const int32_t* assign_slot, const float* assign_w,
                           const int32_t* shared_slot, const uint32_t* deferred, const float* bias, float* out,
                           uint32_t n_tokens, uint32_t hidden, hipStream_t s) {
-    const uint64_t n = (uint64_t)n_tokens * hidden;
-    if (n == 0) return hipSuccess;
-    combine_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(eo, assign_slot, assign_w, shared_slot, deferred, bias,
-                                                               out, n_tokens, hidden);
+    if (n_tokens == 0 || hidden == 0) return hipSuccess;
+    const bool vec = hidden % 4 == 0 && (reinterpret_cast<uintptr_t>(eo) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+    const uint32_t per = vec ? 1024 : 256;
+    const dim3 grid((hidden + per - 1) / per, n_tokens);
+    if (vec)
+        combine_kernel<4><<<grid, 256, 0, s>>>(eo, assign_slot, assign_w, shared_slot, deferred, bias, out, hidden);
+    else
+        combine_kernel<1><<<grid, 256, 0, s>>>(eo, assign_slot, assign_w, shared_slot, deferred, bias, out, hidden);
     return hipGetLastError();
 }
 
