@@ -52,7 +52,6 @@ __global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(Gem
     if (EXPERTS) {  // item-major: the items of one expert follow each other
         item = r8 / a.groups8;
         tg = (r8 % a.groups8) * 8 + xcd;
-        if (item >= *a.n_work) return;
     } else {
         item = r8 % a.n_items;
         tg = (r8 / a.n_items) * 8 + xcd;
@@ -62,7 +61,12 @@ __global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(Gem
     uint32_t first, count;
     uint64_t mat, mat2;
     if (EXPERTS) {
-        const QmmWork w = a.work[item];
+        // The count and the item in one round trip (the grid stays within
+        // the list).
+        uint32_t n_work = *a.n_work;
+        QmmWork w = a.work[item];
+        asm volatile("" : "+s"(n_work), "+s"(w.mat), "+s"(w.slot), "+s"(w.count), "+s"(w.pad));
+        if (item >= n_work) return;
         first = w.slot;
         count = w.count;
         mat = w.mat;
@@ -87,15 +91,19 @@ __global__ __launch_bounds__(KS * 64, MT == 1 ? 4 : 2) void gemm_tile_kernel(Gem
         for (int j = 0; j < NJ; ++j) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     TileStream<FMT, MT, NJ, GU, EXPERTS> st;
-    st.init(a, first, count, mat, mat2, tg, lane);
+    st.init_w(a, mat, mat2, tg, lane);
     uint8_t* const xs = lds + wave * kX;
     const uint32_t s0 = a.turns * wave / KS, s1 = a.turns * (wave + 1) / KS;
     if (s0 < s1) {
+        // The weights first: the rows of x wait for their list.
         st.load_d(s0, s1);
-        st.load_x(s0, s1, 0);
         st.load_w(s0, s1, 0);
-        st.load_x(s0, s1, 1);
         if (FMT == kFmtQ8) st.load_w(s0, s1, 1);
+    }
+    st.init_x(a, first, count, lane);
+    if (s0 < s1) {
+        st.load_x(s0, s1, 0);
+        st.load_x(s0, s1, 1);
     }
     if (FMT == kFmtIq2) lds_barrier();
     for (uint32_t s = s0; s < s1; ++s) {

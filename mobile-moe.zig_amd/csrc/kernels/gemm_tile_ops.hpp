@@ -179,11 +179,24 @@ struct TileStream {
     uint32_t x_voff[kXRows];
     uint32_t rec_voff, col_lane, tile0, tiles, units, cols;
 
-    __device__ __forceinline__ void init(const GemmTileArgs& a, uint32_t first, uint32_t count, uint64_t mat,
-                                         uint64_t mat2, uint32_t tg, uint32_t lane) {
-        x_r = make_rsrc(a.x, a.x_bytes);
+    __device__ __forceinline__ void init_w(const GemmTileArgs& a, uint64_t mat, uint64_t mat2, uint32_t tg,
+                                           uint32_t lane) {
         rec_r = make_rsrc(a.recs + mat * a.rec_stride, (uint32_t)(a.rec_stride * 16));
         if (GU) rec2_r = make_rsrc(a.recs + mat2 * a.rec_stride, (uint32_t)(a.rec_stride * 16));
+        rec_voff = lane * 16;
+        tile0 = tg * kRowTiles;
+        tiles = a.tiles;
+        units = a.units;
+        // Tiles past the matrix read its last tile's scales (their weights
+        // read as zeros).
+        const uint32_t j = min(lane >> 4, NJ - 1u);
+        const uint32_t t = min(tile0 + j % kRowTiles, tiles - 1);
+        d_lane = a.dvals + (j >= kRowTiles ? mat2 : mat) * a.d_stride + (uint64_t)(t * 16 + (lane & 15)) * a.d_row;
+    }
+    __device__ __forceinline__ void init_x(const GemmTileArgs& a, uint32_t first, uint32_t count, uint32_t lane) {
+        x_r = make_rsrc(a.x, a.x_bytes);
+        col_lane = lane % kRowLanes * (64 / kRowLanes);
+        cols = a.cols;
         // Rows past the item read zeros (no memory access).
 #pragma unroll
         for (int i = 0; i < kXRows; ++i) {
@@ -193,17 +206,6 @@ struct TileStream {
             if (a.x_row) row = a.x_row[row];
             x_voff[i] = ok ? row * (a.x_stride * 4) + lane % kRowLanes * 16 : kBufOob;
         }
-        rec_voff = lane * 16;
-        col_lane = lane % kRowLanes * (64 / kRowLanes);
-        tile0 = tg * kRowTiles;
-        tiles = a.tiles;
-        units = a.units;
-        cols = a.cols;
-        // Tiles past the matrix read its last tile's scales (their weights
-        // read as zeros).
-        const uint32_t j = min(lane >> 4, NJ - 1u);
-        const uint32_t t = min(tile0 + j % kRowTiles, tiles - 1);
-        d_lane = a.dvals + (j >= kRowTiles ? mat2 : mat) * a.d_stride + (uint64_t)(t * 16 + (lane & 15)) * a.d_row;
     }
 
     // Half h of turn s; a turn at or past `end` loads nothing (zeros, no
