@@ -62,6 +62,11 @@ struct RouteArgs {
     QmmWork* work_dn;
     uint32_t* n_work;           // [2]: active items of work_gu, work_dn
     uint32_t inter;             // routed expert width (up column offset)
+};
+
+// The routing launch's own arguments (the decode kernels take RouteArgs too and
+// need none of these).
+struct RouteBatchArgs : RouteArgs {
     uint32_t item_rows = kQmmTokens;  // n_tokens > 1: most rows of an item
     uint64_t* tok = nullptr;    // n_tokens > 1: [n_tokens] routed tokens between workgroups
     uint32_t* ticket = nullptr; //               workgroups that have routed, 0 between calls
@@ -319,7 +324,7 @@ hipError_t launch_quantize_silu(const float* src, uint64_t src_stride, uint64_t 
 // Scheduler.route (scheduler.zig:169-262) for every token on the device, plus
 // the problem lists of the expert products.
 
-hipError_t launch_route(const RouteArgs& a, hipStream_t s);
+hipError_t launch_route(const RouteBatchArgs& a, hipStream_t s);
 // Upper bound of the grouped items per list for T tokens and E experts.
 uint32_t route_max_work(uint32_t n_tokens, uint32_t n_experts, uint32_t item_rows);
 

@@ -43,7 +43,7 @@ struct RouteLds {
 
 // Routes this workgroup's tokens; true in the workgroup that ends last, with
 // every token's word in L.tok.
-__device__ bool route_tokens(const RouteArgs& a, RouteLds& L) {
+__device__ bool route_tokens(const RouteBatchArgs& a, RouteLds& L) {
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t T = a.n_tokens, E = a.n_experts, k = a.k;
     const uint32_t n_wg = (T + kRouteTokens - 1) / kRouteTokens;
@@ -101,7 +101,7 @@ __device__ bool route_tokens(const RouteArgs& a, RouteLds& L) {
     return true;
 }
 
-__device__ void route_layout(const RouteArgs& a, RouteLds& L) {
+__device__ void route_layout(const RouteBatchArgs& a, RouteLds& L) {
     uint32_t* const s_cnt = L.cnt;
     uint32_t* const s_rec = L.rec;
     uint32_t* const s_off = L.off;
@@ -198,7 +198,7 @@ __device__ void route_layout(const RouteArgs& a, RouteLds& L) {
     }
 }
 
-__global__ __launch_bounds__(kRouteThreads) void route_kernel(RouteArgs a) {
+__global__ __launch_bounds__(kRouteThreads) void route_kernel(RouteBatchArgs a) {
     __shared__ RouteLds L;
     const uint32_t n_wg = (a.n_tokens + kRouteTokens - 1) / kRouteTokens;
     if (blockIdx.x >= n_wg) {
@@ -267,7 +267,7 @@ uint32_t route_max_work(uint32_t n_tokens, uint32_t n_experts, uint32_t item_row
     return 2 * chunks;
 }
 
-hipError_t launch_route(const RouteArgs& a, hipStream_t s) {
+hipError_t launch_route(const RouteBatchArgs& a, hipStream_t s) {
     if (a.n_tokens < 2 || a.n_tokens > kMaxTokens || a.n_experts > kMaxExperts || a.k == 0 || a.k > kMaxK ||
         a.k > a.n_experts)
         return hipErrorInvalidValue;

@@ -142,8 +142,6 @@ size_t carve(mmhip_moe_layer* L, char* base) {
     L->shared_slot = (int32_t*)take(T * 4);
     L->deferred = (uint32_t*)take(T * 4);
     L->slot_tok = (uint32_t*)take(S * 4);
-    L->route_tok = (uint64_t*)take(T * 8);
-    L->route_ticket = (uint32_t*)take(4);
     L->gemv_gu = (uint4*)take(10 * 16);
     L->gemv_dn = (uint4*)take(5 * 16);
     L->n_gemv = (uint32_t*)take(2 * 4);
@@ -158,7 +156,6 @@ size_t carve(mmhip_moe_layer* L, char* base) {
     L->xq_h = take(quant_act_bytes(T, L->gu->geom.cols_pad));
     L->xq_d = take(quant_act_bytes(S, L->dn->geom.cols_pad));
     if (L->has_shared && !L->shared_merged) L->xq_sd = take(quant_act_bytes(T, L->sh_dn->geom.cols_pad));
-    L->xp = (float*)take(T * H * 4);
     L->bias = (float*)take(H * 4);
     L->dm_hq = (uint8_t*)take(5 * (uint64_t)(I / 32) * 64);
     L->dm_hs = (float*)take(5 * (uint64_t)(I / 32) * 4);
@@ -166,6 +163,11 @@ size_t carve(mmhip_moe_layer* L, char* base) {
     L->dm_flags = (uint32_t*)take(5 * (uint64_t)(I / 32) * 4);
     L->d_in = (float*)take(T * H * 4);
     L->d_out = (float*)take(T * H * 4);
+    // Last: ahead of the decode words above these shifted them, and the
+    // one-launch decode took 2% longer.
+    L->route_tok = (uint64_t*)take(T * 8);
+    L->route_ticket = (uint32_t*)take(4);
+    L->xp = (float*)take(T * H * 4);
     return off;
 }
 
@@ -217,17 +219,17 @@ int check_hip(hipError_t e, const char* what) { return e == hipSuccess ? MMHIP_O
 // Q8_0 experts always (layer of 64 experts of 1536, hidden 2048: 2 tokens 47.0
 // -> 32.3 us, 64 tokens 138 -> 91, 256 tokens 396 -> 188). IQ2_XXS experts keep
 // the digit kernel's 8-row items where a large layer's call has enough of them
-// for its 1024-thread workgroups but few rows each: fewer than the experts, a
-// fifth of an item's cost is then the 16-row tile's empty rows (same layer, 16
-// tokens 46.7 us against 48.0, 48 tokens 62.6 against 66.6, 64 tokens 71.1
-// against 71.4, 256 tokens 158 against 147; 4 tokens, below those workgroups,
-// 49.2 against 39.1; hidden 1024, experts of 512: 64 tokens 39.3 against 31.0). A
+// for its 1024-thread workgroups but no more tokens than experts, so that the
+// 16-row tile would be mostly empty rows (same layer, 16 tokens 46.7 us against
+// 48.0, 48 tokens 62.6 against 66.6, 64 tokens 70.6 against 71.4 to 73.2, 96
+// tokens 86.0 against 84.6, 256 tokens 158 against 147; 4 tokens, below those
+// workgroups, 49.2 against 39.1; hidden 1024, experts of 512: 64 tokens 39.3 against 31.0). A
 // separate shared expert costs the digit path five launches (92.6 us against
 // 79.6 at 64 tokens).
 bool moe_tile(const mmhip_moe_layer* L, uint32_t T, int num_cu) {
     if (T == 1) return false;
     const TileGeom& g = L->gu->geom;
-    if (g.fmt == kFmtIq2 && !L->sh_gu && T < L->n_experts && (uint64_t)L->inter * L->hidden >= (1u << 21) &&
+    if (g.fmt == kFmtIq2 && !L->sh_gu && T <= L->n_experts && (uint64_t)L->inter * L->hidden >= (1u << 21) &&
         group_large(g, route_max_work(T, L->n_experts, kQmmTokens), num_cu))
         return false;
     if (!gemm_tile_fits(L->gu->geom, T, L->hidden) || !gemm_tile_fits(L->dn->geom, 5 * T, L->inter)) return false;
@@ -240,7 +242,7 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
                 bool with_bias, uint32_t* route_ids, float* route_w) {
     const uint32_t H = L->hidden, I = L->inter, E = L->n_experts;
     hipStream_t s = ctx->stream;
-    RouteArgs r{};
+    RouteBatchArgs r{};
     r.scores = L->scores;
     r.n_tokens = T;
     r.n_experts = E;
