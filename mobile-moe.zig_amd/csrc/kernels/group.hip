@@ -1,7 +1,10 @@
-// Quantised matmul over groups of 8 activation rows on gfx950: prompt prefill
-// (qmm.matMulQ8_0's role, qmm.zig:58-138) and the MoE experts of a batch
-// grouped by expert (moeFFN over forwardBatch's tokens, inference.zig:346-351,
-// 886-1188).
+// Quantised matmul over groups of 8 activation rows on gfx950: the MoE experts
+// of a batch grouped by expert (moeFFN over forwardBatch's tokens,
+// inference.zig:346-351, 886-1188) in large IQ2_XXS layers whose experts get few
+// rows each, and small Q8_0 prompt calls (qmm.matMulQ8_0's role, qmm.zig:58-138).
+// Other calls run on the bf16 matrix cores (gemm_tile.hip); the dense form of
+// group_kernel takes only inputs of 2 GiB and more, which that kernel's 32-bit
+// offsets do not reach.
 //
 // An item is one weight matrix and up to 8 activation rows: consecutive rows
 // of a batch (dense) or the slots of one expert (grouped, items written by the
