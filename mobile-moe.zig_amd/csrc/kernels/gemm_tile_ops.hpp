@@ -248,22 +248,23 @@ struct TileStream {
     __device__ __forceinline__ void scales(float (&c)[4][4]) const {
         if constexpr (FMT == kFmtIq2) {
             const uint32_t g = (threadIdx.x & 63) >> 4;
-            // (0.5 + ls) / 4 = ls (2 / 8) + 1 / 8 of the row's scale (dequant.zig:336).
-            float d8[4], d2[4];
+            // (0.5 + ls) / 4 = (2 ls + 1) / 8 of the row's scale (dequant.zig:336),
+            // as one product: ls (2 / 8) + 1 / 8 is a NaN for an infinite
+            // scale and ls = 0.
+            float d8[4];
             broadcast_rows4(f16_scale((uint16_t)d.x) * (0.125f * kActUnscale), d8);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) d2[j] = d8[j] * 2.0f;
-#pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                // Byte b: ls of sub-block b of the half unit, gathered from
-                // the row's four lane groups.
-                const uint32_t mine = ((iq[j].x >> 30) | ((iq[j].y >> 30) << 2)) << (8 * g);
+                // Byte b: 2 ls + 1 of sub-block b of the half unit, gathered
+                // from the row's four lane groups.
+                const uint32_t ls2 = ((iq[j].x >> 29) & 6u) | ((iq[j].y >> 27) & 0x18u) | 1u;
+                const uint32_t mine = ls2 << (8 * g);
                 const auto p = __builtin_amdgcn_permlane16_swap(mine, mine, false, false);
                 const uint32_t pair = p[0] | p[1];
                 const auto q = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
                 const uint32_t ls = q[0] | q[1];
 #pragma unroll
-                for (int b = 0; b < 4; ++b) c[b][j] = fmaf((float)((ls >> (8 * b)) & 0xFFu), d2[j], d8[j]);
+                for (int b = 0; b < 4; ++b) c[b][j] = (float)((ls >> (8 * b)) & 0xFFu) * d8[j];
             }
         } else {
 #pragma unroll

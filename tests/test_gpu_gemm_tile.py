@@ -65,3 +65,17 @@ def test_extreme_vectors(ctx, orc, fmt):
     y = ctx.batch_mat_mul(raw, fmt, x, rows, batch, cols)
     _check(y[[0, 2, 4]], x[[0, 2, 4]], w)
     assert np.all(np.isnan(y[[1, 3]]))
+
+
+def test_infinite_block_scale(ctx, orc):
+    """IQ2_XXS superblocks of infinite scale, sub-block scale codes of zero among
+    them, times vectors of the weights' signs: every product is +inf, and so is
+    the sum (the CPU path's result, dequant.zig:316-355)."""
+    rng = np.random.default_rng(78)
+    rows, cols = 16, 768
+    raw = mm.make_iq2_xxs(rng, rows, cols).reshape(rows, cols // 256, 66)
+    raw[:, :, :2] = np.array([0x3C00], np.uint16).view(np.uint8)  # 1.0
+    signs = np.sign(orc.dequantize(raw.reshape(-1), mm.IQ2_XXS, rows * cols)).reshape(rows, cols).astype(np.float32)
+    raw[:, 1, :2] = np.array([0x7C00], np.uint16).view(np.uint8)  # inf
+    y = ctx.batch_mat_mul(raw.reshape(-1), mm.IQ2_XXS, signs, rows, rows, cols)
+    assert np.all(np.diagonal(y) == np.inf)
