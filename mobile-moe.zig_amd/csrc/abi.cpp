@@ -39,16 +39,31 @@ bool gfx950_present(int* count_out) {
     return false;
 }
 
-// Resident weight for a host pointer (getOrUploadMatBuffer semantics).
-// Host calls. Results up to 1 MiB go straight to the pinned host buffer, as
-// the kernels write every output once: a copy behind the kernel costs its own
-// launch (Q8_0 [1536 x 2048] times one vector 22.1 -> 20.5 us, [8192 x 4096] 34.4
-// -> 24.7; at 2 MiB the two are within a run's spread). Inputs of 32 KiB to 512
-// KiB are copied by a kernel, which starts without the copy engine's hand-over
-// (64 KiB 36.1 -> 33.8 us a call, 256 KiB 68.1 -> 63.3); below, the runtime's
-// copy is as fast, at 1 MiB faster (190 against 196).
+// Host calls. Results up to 1 MiB go straight to the pinned host buffer: a copy
+// behind the kernel costs its own launch (Q8_0 [1536 x 2048] times one vector
+// 22.1 -> 20.5 us, [8192 x 4096] 34.4 -> 24.7; at 2 MiB the two are within a run's
+// spread). Inputs of 32 KiB to 512 KiB are copied by a kernel, which starts
+// without the copy engine's hand-over (64 KiB 36.1 -> 33.8 us a call, 256 KiB
+// 68.1 -> 63.3); below, the runtime's copy is as fast, at 1 MiB faster (190
+// against 196).
 constexpr uint64_t kKernelCopyMin = 32u << 10, kKernelCopyMax = 512u << 10, kDirectOutMax = 1u << 20;
 
+bool direct_results(const mmhip_ctx* ctx, const mmhip_weight* w, uint64_t batch) {
+    const uint64_t words = batch * w->rows;
+    if (words > kDirectOutMax / 4) return false;
+    if (w->type != kF32 && w->type != kF16) return true;
+    if (batch > 1 && gemm_strict_fits((uint32_t)batch, (uint32_t)w->rows, (uint32_t)w->cols, w->cols, ctx->num_cu))
+        return true;
+    // The float row kernels store single words, about 1.3 ns each over the
+    // link; a copy costs 1.6 us up to 16 KiB and 10 us past that. Direct and
+    // copied, us, f32: [2048 x 512] 22.6 and 22.6, [4096 x 512] 26.1 and 24.3,
+    // [256 x 512] times 16 25.2 and 23.1, [6144 x 512] 29.8 and 32.0, [16384 x
+    // 256] 45.2 and 38.2, [32768 x 256] 63.3 and 50.1; from 1024 columns on the
+    // weights' reads hide the stores, [16384 x 1024] 43.3 and 47.3.
+    return words <= 2048 || (words > 4096 && (words <= 8192 || w->cols >= 1024));
+}
+
+// Resident weight for a host pointer (getOrUploadMatBuffer semantics).
 int resident_weight(mmhip_ctx* ctx, const void* ptr, uint32_t type, uint64_t rows, uint64_t cols,
                     mmhip_weight** out) {
     auto key = std::make_tuple(ptr, type, rows, cols);
@@ -277,7 +292,7 @@ int mmhip_batch_mat_mul(mmhip_ctx* ctx, float* out, const void* ptr, uint32_t ty
     if (rc) return rc;
     const size_t in_bytes = batch * in_dim * 4, out_bytes = batch * out_dim * 4;
     const bool in_kernel = in_bytes >= kKernelCopyMin && in_bytes <= kKernelCopyMax;
-    const bool out_direct = out_bytes <= kDirectOutMax;
+    const bool out_direct = direct_results(ctx, w, batch);
     hipError_t e = ctx->h_in.ensure(in_bytes);
     if (e == hipSuccess) e = ctx->h_out.ensure(out_bytes);
     if (e == hipSuccess) e = ctx->d_in.ensure(in_bytes);

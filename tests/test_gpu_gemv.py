@@ -276,6 +276,43 @@ def test_seam_batches_by_size(ctx, orc, rows, cols, batch):
         assert np.array_equal(y[b].view(np.uint32), one.view(np.uint32))
 
 
+@pytest.mark.parametrize("t", [mm.F32, mm.F16])
+@pytest.mark.parametrize("rows,cols,batch", [(2048, 12, 1), (2049, 12, 1), (4096, 12, 1), (4097, 12, 1), (8193, 12, 1),
+                                             (8193, 1024, 1), (256, 12, 16), (128, 12, 16)])
+def test_seam_float_results_by_size(ctx, orc, t, rows, cols, batch):
+    """Host calls on both sides of every size at which single-word results go
+    to the host by a copy or straight from the kernel: the CPU path's bits."""
+    rng = np.random.default_rng(rows + cols + batch)
+    raw = _weights(rng, t, rows, cols)
+    for _ in range(2):  # other vectors through the same buffers
+        x = rng.standard_normal((batch, cols)).astype(np.float32)
+        ref = orc.batch_mat_mul_unified(raw, t, x, rows, batch, cols)
+        _bits_equal(ctx.batch_mat_mul(raw, t, x, rows, batch, cols).reshape(-1), np.asarray(ref).reshape(-1))
+
+
+@pytest.mark.parametrize("rows,cols,batch", [(33, 2330, 13), (700, 4100, 2), (40, 330, 17)])
+def test_seam_ragged_q8_batches(ctx, orc, rows, cols, batch):
+    """Host calls with a partial last Q8_0 block, below and above the 2048
+    columns whose sums a kernel keeps to itself: the oracle's results, and the
+    device call's bits."""
+    rng = np.random.default_rng(rows + cols + batch)
+    raw = _weights(rng, mm.Q8_0, rows, cols)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    y = ctx.batch_mat_mul(raw, mm.Q8_0, x, rows, batch, cols)
+    ref = orc.batch_mat_mul_unified(raw, mm.Q8_0, x, rows, batch, cols).reshape(batch, rows)
+    assert mm.max_abs_rel(y, ref) <= TOL_QMM
+    w = ctx.upload(raw, mm.Q8_0, rows, cols)
+    dx, dy = mm.DeviceArray.from_numpy(ctx, x), mm.DeviceArray(ctx, rows * batch * 4)
+    try:
+        ctx.qmm_dev(w, 0, dx, dy, batch)
+        ctx.synchronize()
+        dev = dy.to_numpy(np.float32, batch * rows)
+    finally:
+        for h in (w, dx, dy):
+            h.free()
+    assert np.array_equal(dev.view(np.uint32), y.reshape(-1).view(np.uint32))
+
+
 def test_seam_is_thread_safe(ctx, orc):
     """The reference re-enters the seam from 4 pool workers at once
     (inference.zig:934-971); 4 threads must get the same answers as 1."""
