@@ -67,6 +67,26 @@ def test_extreme_vectors(ctx, orc, fmt):
     assert np.all(np.isnan(y[[1, 3]]))
 
 
+@pytest.mark.parametrize("exp", [-104, -112, -120])
+@pytest.mark.parametrize("fmt", [mm.Q8_0, mm.IQ2_XXS])
+def test_tiny_vectors(ctx, orc, fmt, exp):
+    """Below 2^-105 an element's second part is a subnormal bf16 number: off by at
+    most 2^-134, which the 2^-12 that vectors enter with makes 2^-122."""
+    rng = np.random.default_rng(79 + fmt - exp)
+    rows, cols, batch = 40, 2304, 5
+    raw = mm.make_weight(rng, fmt, rows, cols)
+    w = orc.dequantize(raw, fmt, rows * cols).reshape(rows, cols).astype(np.float64)
+    x = np.ldexp(rng.uniform(0.5, 1.0, (batch, cols)) * rng.choice([-1.0, 1.0], (batch, cols)), exp).astype(np.float32)
+    y = ctx.batch_mat_mul(raw, fmt, x, rows, batch, cols)
+    x64 = x.astype(np.float64)
+    err = np.abs(y.astype(np.float64) - x64 @ w.T)
+    off = np.maximum(2.0 ** -17 * np.abs(x64), 2.0 ** -122)
+    # The f32 sums as in the bound above, and half a smallest f32 per output block.
+    bound = (off + (cols + 16) * 2.0 ** -24 * np.abs(x64)) @ np.abs(w).T + cols * 2.0 ** -149
+    print(f"error / bound at most {float((err / bound).max()):.3f}")
+    assert np.all(err <= bound)
+
+
 def test_infinite_block_scale(ctx, orc):
     """IQ2_XXS superblocks of infinite scale, sub-block scale codes of zero among
     them, times vectors of the weights' signs: every product is +inf, and so is

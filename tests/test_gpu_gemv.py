@@ -218,7 +218,7 @@ def test_qmm_q8_every_k_split(ctx, orc, cols):
     """Q8_0 matmul over every K width the one-launch kernel splits its own
     way (units of 64 columns per 16-row tile: 4 -> one slice, 12 -> three
     one-step slices, 16 -> two, 20 -> five, 24 -> three two-step slices,
-    28 -> seven, 32 -> four) and one past it (2304: the two-launch path),
+    28 -> seven, 32 -> four) and one past it (2304: the bf16 tile kernel),
     with a ragged batch and ragged rows, both output layouts, against the
     oracle's matMulQ8_0 (qmm.zig:58-138)."""
     rng = np.random.default_rng(cols)
@@ -236,6 +236,30 @@ def test_qmm_q8_every_k_split(ctx, orc, cols):
             y = dy.to_numpy(np.float32, rows * batch)
             y = y.reshape(batch, rows).T if layout == 0 else y.reshape(rows, batch)
             assert mm.max_abs_rel(y, ref_mn) <= TOL_QMM, (cols, layout)
+    finally:
+        w.free()
+        dx.free()
+        dy.free()
+
+
+@pytest.mark.parametrize("rows,cols,batch", [(33, 40, 2), (100, 330, 13), (17, 2047, 65), (50, 2330, 8), (16, 4100, 9)])
+def test_qmm_q8_partial_blocks(ctx, orc, rows, cols, batch):
+    """Q8_0 rows that end in a partial block: digits of the vectors in scratch,
+    then the grouped kernel, below and above one 2048-column chunk, both layouts."""
+    rng = np.random.default_rng(rows + cols + batch)
+    raw = _weights(rng, mm.Q8_0, rows, cols)
+    xin = rng.standard_normal((batch, cols)).astype(np.float32)
+    ref = orc.batch_mat_mul_unified(raw, mm.Q8_0, xin, rows, batch, cols).reshape(batch, rows)
+    w = ctx.upload(raw, mm.Q8_0, rows, cols)
+    dx = mm.DeviceArray.from_numpy(ctx, xin)
+    dy = mm.DeviceArray(ctx, rows * batch * 4)
+    try:
+        for layout in (0, 1):
+            ctx.qmm_dev(w, 0, dx, dy, batch, layout)
+            ctx.synchronize()
+            y = dy.to_numpy(np.float32, rows * batch)
+            y = y.reshape(batch, rows) if layout == 0 else y.reshape(rows, batch).T
+            assert mm.max_abs_rel(y, ref) <= TOL_GEMV, layout
     finally:
         w.free()
         dx.free()
@@ -263,10 +287,11 @@ def test_qmm_reference_kats(ctx, orc):
         assert np.all(np.abs(exp - out[ni]) <= 0.01)
 
 
-@pytest.mark.parametrize("rows,cols,batch", [(3, 2731, 3), (5, 2730, 3), (700, 512, 400), (16, 4099, 32), (16, 4097, 32)])
+@pytest.mark.parametrize("rows,cols,batch", [(3, 2731, 3), (5, 2730, 3), (4, 4097, 2), (4, 2733, 3), (700, 512, 400),
+                                             (16, 4099, 32), (16, 4097, 32), (16, 4096, 32)])
 def test_seam_batches_by_size(ctx, orc, rows, cols, batch):
     """Host calls whose vectors or results lie at the sizes where the copies
-    change: every output is the single-vector call's, bit for bit."""
+    change (vectors: 32 and 512 KiB, with every remainder of 16 bytes): every output is the single-vector call's, bit for bit."""
     rng = np.random.default_rng(rows + cols)
     raw = rng.standard_normal((rows, cols)).astype(np.float32)
     x = rng.standard_normal((batch, cols)).astype(np.float32)

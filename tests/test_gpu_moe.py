@@ -236,6 +236,61 @@ def test_iq2_expert_groups_large_layer(ctx, orc, t, n_exp, inter):
         gpu.free()
 
 
+@pytest.mark.parametrize("t", [33, 100, 256])
+@pytest.mark.parametrize("fmt,hidden,inter,shared_inter", [(mm.Q8_0, 288, 96, 1504), (mm.IQ2_XXS, 256, 256, 1536)])
+def test_separate_shared_expert_tiles(ctx, orc, t, fmt, hidden, inter, shared_inter):
+    """A separate shared expert wide enough for each larger tile of its gate, up
+    and activation launch (256 CUs: 16x64 at 33 tokens, 32x64 by eight waves at
+    100, by four at 256; whole columns make its row tiles an even number)."""
+    rng = np.random.default_rng(400 + t + fmt)
+    E = 5
+    router, gate, up, down, shared = _weights(rng, fmt, hidden, inter, E, shared_inter=shared_inter, router_sigma=0.05)
+    gpu, cpu = _layers(ctx, orc, fmt, hidden, inter, E, router, gate, up, down, shared, shared_inter=shared_inter)
+    try:
+        h = rng.standard_normal((t, hidden)).astype(np.float32)
+        out_g, ids_g, w_g = gpu.ffn(h)
+        out_c, ids_c, w_c = cpu.ffn(h)
+        assert _check(orc, router, h, out_g, ids_g, w_g, out_c, ids_c, w_c) < 1e-4
+    finally:
+        gpu.free()
+
+
+@pytest.mark.parametrize("t", [2, 17, 90])
+@pytest.mark.parametrize("hidden,inter,shared_inter", [(330, 200, None), (330, 200, 200), (330, 192, 200), (320, 200, 96)])
+def test_q8_experts_of_partial_blocks(ctx, orc, t, hidden, inter, shared_inter):
+    """Q8_0 experts whose rows end in a partial block (hidden, inter or both)
+    stay on the digit kernels, with each kind of shared expert. The reference
+    finds an expert by its elements' blocks, which whole blocks only give, so the
+    experts' products are formed here in float64 (expertFFN,
+    inference.zig:1152-1188) on the oracle's routing."""
+    rng = np.random.default_rng(410 + t + inter)
+    E = 6
+    router, gate, up, down, shared = _weights(rng, mm.Q8_0, hidden, inter, E, shared_inter=shared_inter, router_sigma=0.05)
+    gpu, cpu = _layers(ctx, orc, mm.Q8_0, hidden, inter, E, router, gate, up, down, shared, shared_inter=shared_inter)
+
+    def mats(raw, rows, cols, n):
+        wide = (cols + 31) // 32 * 32
+        return orc.dequantize(raw, mm.Q8_0, n * rows * wide).reshape(n, rows, wide)[:, :, :cols].astype(np.float64)
+
+    def ffn(x, g, u, d):
+        a = g @ x
+        return d @ (a / (1 + np.exp(-a)) * (u @ x))
+
+    try:
+        h = rng.standard_normal((t, hidden)).astype(np.float32)
+        out_g, ids_g, w_g = gpu.ffn(h)
+        _, ids_c, w_c = cpu.ffn(h)
+    finally:
+        gpu.free()
+    g, u, d = mats(gate, inter, hidden, E), mats(up, inter, hidden, E), mats(down, hidden, inter, E)
+    sh = shared and [m[0] for m in (mats(shared[0], shared_inter, hidden, 1), mats(shared[1], shared_inter, hidden, 1),
+                                    mats(shared[2], hidden, shared_inter, 1))]
+    x = h.astype(np.float64)
+    ref = np.array([sum(w_c[i, j] * ffn(x[i], g[e], u[e], d[e]) for j, e in enumerate(ids_c[i])) +
+                    (ffn(x[i], *sh) if sh else 0.0) for i in range(t)])
+    _check(orc, router, h, out_g, ids_g, w_g, ref, ids_c, w_c)
+
+
 @pytest.mark.parametrize("t", [1, 6])
 @pytest.mark.parametrize("variant", ["wider", "other_type", "none"])
 def test_shared_expert_variants(ctx, orc, t, variant):

@@ -3,8 +3,9 @@ with the library's fixed per-device scratch instead of an allocated one.
 
 Its output must equal mmhip_qmm_dev's bit for bit (same kernels, same
 inputs) on two calls in a row, the second with a smaller input, so that
-nothing left in the shared scratch by the first call leaks into the second;
-both are also checked against the oracle's matMulQ8_0 / dequantize + GEMV
+nothing left in the shared scratch by the first call leaks into the second
+(only Q8_0 rows that end in a partial block use the scratch; the others run in
+one launch without it); both are also checked against the oracle's matMulQ8_0 / dequantize + GEMV
 (qmm.zig:58-138, inference.zig:1231-1264) at the QMM tolerance. Inputs beyond
 the fixed scratch are refused with an error.
 """
@@ -48,6 +49,26 @@ def test_noalloc_matches_qmm_dev_twice(ctx, orc, fmt, layout):
         assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (rows, cols, batch)
         cpu = orc.batch_mat_mul_unified(raw, fmt, x, rows, batch, cols).reshape(batch, rows)
         assert mm.max_abs_rel(got, cpu) <= TOL_QMM
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+def test_noalloc_scratch_holds_nothing_over(ctx, orc, layout):
+    """Q8_0 rows that end in a partial block, whose digits go through the fixed
+    scratch: a call that fills it to the last byte (256 vectors of 8190 columns),
+    then smaller ones, each with mmhip_qmm_dev's bits and the oracle's results."""
+    rng = np.random.default_rng(940 + layout)
+    for rows, cols, batch in [(48, 8190, 256), (100, 1000, 7), (33, 2330, 64), (16, 40, 2)]:
+        raw = mm.make_weight(rng, mm.Q8_0, rows, cols)
+        x = (rng.standard_normal((batch, cols)) * 2.0).astype(np.float32)
+        w = ctx.upload(raw, mm.Q8_0, rows, cols)
+        try:
+            got = _run(ctx, ctx.qmm_dev_noalloc, w, x, rows, batch, layout)
+            ref = _run(ctx, ctx.qmm_dev, w, x, rows, batch, layout)
+        finally:
+            w.free()
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (rows, cols, batch)
+        cpu = orc.batch_mat_mul_unified(raw, mm.Q8_0, x, rows, batch, cols).reshape(batch, rows)
+        assert mm.max_abs_rel(got, cpu) <= 1e-3
 
 
 def test_noalloc_size_limit(ctx):
