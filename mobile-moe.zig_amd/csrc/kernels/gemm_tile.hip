@@ -255,7 +255,10 @@ GemmTileArgs base(const uint4* recs, const uint16_t* dvals, const TileGeom& g, c
 }  // namespace
 
 bool gemm_tile_fits(const TileGeom& g, uint64_t x_rows, uint64_t x_stride) {
-    return g.cols % 32 == 0 && x_rows > 0 && x_stride >= g.cols && x_rows <= 0x7FFFFFFFu / 4 / x_stride;
+    if (g.cols % 32 || x_rows == 0 || x_stride < g.cols || x_rows > 0x7FFFFFFFu / 4 / x_stride) return false;
+    // A launch of 2^32 threads or more does not run: the largest dense calls are
+    // 32x64 tiles of 256 threads (3.4e10 results, 137 GB).
+    return (g.tiles / 4 + 8) * ((x_rows + 31) / 32) < 1u << 24;
 }
 
 hipError_t launch_gemm_tile(const uint4* recs, const uint16_t* dvals, const TileGeom& g, uint64_t mat, bool gate_up,
