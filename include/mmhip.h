@@ -288,7 +288,13 @@ typedef struct {
 int mmhip_gemv_grouped_dev(mmhip_ctx* ctx, const mmhip_gemv_group* groups, uint32_t n_groups);
 /* Batched QMM for prompt prefill: X [batch][cols] -> Y.
  * out_layout 0: Y [batch][rows] (batchMatMulUnified's layout);
- * out_layout 1: Y [rows][batch] (qmm.matMulQ8_0's layout, qmm.zig:52-57). */
+ * out_layout 1: Y [rows][batch] (qmm.matMulQ8_0's layout, qmm.zig:52-57).
+ * The kernel, and with it the number format of the activations and the order of
+ * the sums, is chosen by shape and batch: a call repeated gives the same bits,
+ * but a quantised weight times the same vector in a batch of another size may
+ * differ by the error of the coarser form, about 2e-5 of the result. The same
+ * holds for mmhip_batch_mat_mul and for the tokens of an MoE layer call (about
+ * 1e-4 there). f32 / f16 weights give the same bits at every batch. */
 int mmhip_qmm_dev(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t mat,
                   const float* x_dev, float* y_dev, uint64_t batch,
                   int out_layout);
@@ -296,15 +302,14 @@ int mmhip_qmm_dev(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t mat,
 /* mmhip_qmm_dev without any allocation, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, hosts
  * that forbid hipMalloc). No counterpart in the reference. Same kernels and
- * results as mmhip_qmm_dev; the quantised activations go to a fixed scratch
- * of MMHIP_NOALLOC_SCRATCH_BYTES per device, held until the process ends, so
- * quantised weights need batch x cols256 x 2.125 <= MMHIP_NOALLOC_SCRATCH_BYTES
- * (cols256 = cols rounded up to 256: e.g. 256 rows of 8192 columns), else
- * MMHIP_ERR_INVALID. Calls on one device share that scratch: calls that
- * overlap on a device (two streams, two contexts, two threads) race. Not
- * timed by mmhip_profile_*. f32 / f16 weights use no scratch, nor do Q8_0
- * weights of at most 2048 columns (their activations are quantised inside
- * the one matmul launch; MMHIP_QMM_FUSED=0 turns that off). */
+ * results as mmhip_qmm_dev. Calls of quantised weights are limited to
+ * batch x cols256 x 2.125 <= MMHIP_NOALLOC_SCRATCH_BYTES (cols256 = cols
+ * rounded up to 256: e.g. 256 rows of 8192 columns), else MMHIP_ERR_INVALID,
+ * so that the limit does not depend on the kernel that is chosen. Only Q8_0
+ * weights whose columns are not a multiple of 32 use the scratch itself, for
+ * their quantised activations: it is one per device, held until the process
+ * ends, and such calls that overlap on a device (two streams, two contexts, two
+ * threads) race. All other weights use none. Not timed by mmhip_profile_*. */
 #define MMHIP_NOALLOC_SCRATCH_BYTES 4456448u
 int mmhip_qmm_dev_noalloc(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t mat,
                           const float* x_dev, float* y_dev, uint64_t batch,

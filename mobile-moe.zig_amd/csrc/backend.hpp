@@ -145,7 +145,8 @@ int qmm_device(mmhip_ctx* ctx, const mmhip_weight* w, uint64_t mat, const float*
 // How the batched matmul of w runs: one launch with the activations quantised
 // to int8 digits inside (Q8_0, K <= 2048, small calls), one launch on the bf16
 // matrix cores reading the activations as they are, or two launches through
-// digit scratch (x of 2 GiB and more).
+// digit scratch (what gemm_tile_fits leaves: Q8_0 rows that end in a partial
+// block, x of 2 GiB and more, more than 3.4e10 results).
 enum class QmmPath { kFusedQ8, kTile, kTwoLaunch };
 QmmPath qmm_path(const mmhip_ctx* ctx, const mmhip_weight* w, uint64_t batch);
 

@@ -36,14 +36,18 @@ struct GemmTileArgs {
     uint32_t groups, groups8, n_items;  // set by the launch
 };
 
-// Activations enter the products times 2^-12: 32 products of at most 127 x
-// (127 * 32 < 2^12) then stay finite in f32 for every finite x. The weight
-// scales carry the 2^12.
+// Activations enter the products times 2^-12, so that a block's 32 products of at
+// most 128 x (a code of -128) stay within f32 for every finite x: their sum
+// reaches 2^128 only where the first parts round up to it, and there the second
+// parts, which are summed before them, have the other sign. The weight scales
+// carry the 2^12.
 constexpr float kActScale = 0x1p-12f, kActUnscale = 0x1p12f;
 
 // Four f32 values as two times four bf16: the nearest bf16 and the nearest
-// bf16 to what is left, 16 bits of significand and more (error at most 2^-18
-// of the value; the int8 digit planes give 2^-16 of the block's largest). An
+// bf16 to what is left, 16 bits of significand and more (error at most 2^-17
+// of the value, down to values of 2^-105; below, where the second part is a
+// subnormal number, at most 2^-122; the int8 digit planes give 2^-16 of the
+// block's largest and zeros for blocks below 2^-100). An
 // infinity leaves a NaN in the second part: it poisons its row's outputs, as a
 // NaN does.
 __device__ __forceinline__ void split_bf16(const uint4& q, uint2& hi, uint2& lo) {

@@ -2,9 +2,10 @@
 // of a batch grouped by expert (moeFFN over forwardBatch's tokens,
 // inference.zig:346-351, 886-1188) in large IQ2_XXS layers whose experts get few
 // rows each, and small Q8_0 prompt calls (qmm.matMulQ8_0's role, qmm.zig:58-138).
-// Other calls run on the bf16 matrix cores (gemm_tile.hip); the dense form of
-// group_kernel takes only inputs of 2 GiB and more, which that kernel's 32-bit
-// offsets do not reach.
+// Other calls run on the bf16 matrix cores (gemm_tile.hip), except those that
+// gemm_tile_fits leaves to group_kernel, dense or grouped: Q8_0 rows that end in
+// a partial block, inputs of 2 GiB and more (past that kernel's 32-bit offsets)
+// and dense calls of more than 3.4e10 results.
 //
 // An item is one weight matrix and up to 8 activation rows: consecutive rows
 // of a batch (dense) or the slots of one expert (grouped, items written by the

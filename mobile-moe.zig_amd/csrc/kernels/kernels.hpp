@@ -287,7 +287,8 @@ hipError_t launch_group_experts(const uint4* recs, const uint16_t* dvals, const 
 
 // f32 vectors times quantised weights on the bf16 matrix cores
 // (gemm_tile.hip), the vectors read as they are (columns a multiple of 32,
-// x_rows rows x_stride floats apart, below 2 GiB: gemm_tile_fits).
+// x_rows rows x_stride floats apart, below 2 GiB, at most 3.4e10 results:
+// gemm_tile_fits).
 // y[j * y_slot + r * y_row] = x[j] . W[r]; gate_up: y = silu(x . W_mat[r]) *
 // (x . W_mat+1[r]). Experts: item i < *n_work takes slots [slot, slot +
 // count) (count <= kTileTokens; x row x_row[slot], or the slot itself when

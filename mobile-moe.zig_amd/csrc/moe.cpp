@@ -22,8 +22,9 @@
 //     gate/up       expert-sorted slots times gate and up, and
 //                   silu(gate) * up                         "moe_gateup"
 //     down                                                  "moe_down"
-//   T > 1, other calls of IQ2_XXS experts:
-//     (the routing launch quantises the hidden states)
+//   T > 1, other calls (large IQ2_XXS layers with few tokens per
+//   expert, Q8_0 rows that end in a partial block):
+//     hidden states quantised, IQ2_XXS in the routing launch "moe_quantize"
 //     gate/up       grouped QMM over expert-sorted slots      "moe_gateup"
 //     silu*up       quantised per slot                        "moe_quantize"
 //     down          grouped QMM                               "moe_down"

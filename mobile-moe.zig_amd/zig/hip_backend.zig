@@ -267,8 +267,9 @@ pub const HipBackend = struct {
     /// The batched QMM on device buffers with the library's fixed scratch:
     /// allocates nothing, for code under graph capture or in loops that must
     /// not allocate. No reference counterpart. batch x cols (rounded up to
-    /// 256) x 2.125 bytes must fit the 4,456,448-byte scratch; calls that
-    /// overlap on one device race.
+    /// 256) x 2.125 bytes must fit the 4,456,448-byte scratch; calls with
+    /// Q8_0 columns not a multiple of 32 use it and race where they overlap
+    /// on one device.
     pub fn qmmDevNoAlloc(self: *Self, w: *const Weight, mat: u64, x_dev: [*]const f32, y_dev: [*]f32, batch: u64, out_layout: c_int) !void {
         try check(mmhip_qmm_dev_noalloc(self.ctx, w, mat, x_dev, y_dev, batch, out_layout));
     }
