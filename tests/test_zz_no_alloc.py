@@ -5,10 +5,14 @@ Its output must equal mmhip_qmm_dev's bit for bit (same kernels, same
 inputs) on two calls in a row, the second with a smaller input, so that
 nothing left in the shared scratch by the first call leaks into the second
 (only Q8_0 rows that end in a partial block use the scratch; the others run in
-one launch without it); both are also checked against the oracle's matMulQ8_0 / dequantize + GEMV
-(qmm.zig:58-138, inference.zig:1231-1264) at the QMM tolerance. Inputs beyond
-the fixed scratch are refused with an error.
+one launch without it); both are also checked against the oracle's matMulQ8_0 /
+dequantize + GEMV (qmm.zig:58-138, inference.zig:1231-1264) at the QMM
+tolerance. Inputs beyond the fixed scratch are refused with an error. Captured
+calls (HIP graphs) give the eager calls' bits on every replay, as do an MoE
+layer's.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -101,3 +105,97 @@ def test_noalloc_at_the_limit(ctx, orc):
     finally:
         w.free()
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+def _put(ctx, d, arr):
+    arr = np.ascontiguousarray(arr, dtype=np.float32)
+    mm.check(ctx.lib.mmhip_memcpy_h2d(ctx.handle, d.ptr, mm._ptr(arr), arr.nbytes), "mmhip_memcpy_h2d")
+
+
+class _Graph:
+    """A captured sequence of calls on the context's stream (HIP runtime)."""
+
+    def __init__(self, ctx, calls):
+        self.hip, self.stream = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p(ctx.stream)
+        graph, self.exe = ctypes.c_void_p(), ctypes.c_void_p()
+        self._ok(self.hip.hipStreamBeginCapture(self.stream, 2))  # hipStreamCaptureModeRelaxed
+        try:
+            calls()
+        finally:
+            rc = self.hip.hipStreamEndCapture(self.stream, ctypes.byref(graph))
+        self._ok(rc)
+        self._ok(self.hip.hipGraphInstantiate(ctypes.byref(self.exe), graph, None, None, ctypes.c_size_t(0)))
+        self._ok(self.hip.hipGraphDestroy(graph))
+
+    @staticmethod
+    def _ok(rc):
+        assert rc == 0, f"HIP error {rc}"
+
+    def launch(self):
+        self._ok(self.hip.hipGraphLaunch(self.exe, self.stream))
+
+    def free(self):
+        self._ok(self.hip.hipGraphExecDestroy(self.exe))
+
+
+@pytest.mark.parametrize("fmt,cols", [(mm.Q8_0, 1000), (mm.Q8_0, 768), (mm.Q8_0, 2304), (mm.IQ2_XXS, 768)])
+def test_noalloc_under_capture(ctx, fmt, cols):
+    """A captured call replayed with other vectors each time, eager calls in
+    between: every replay gives the eager call's bits (the scratch, the digit
+    kernel and the tile kernel)."""
+    rng = np.random.default_rng(970 + cols)
+    rows, batch = 100, 19
+    w = ctx.upload(mm.make_weight(rng, fmt, rows, cols), fmt, rows, cols)
+    dx, dy, de = (mm.DeviceArray(ctx, n * 4) for n in (batch * cols, batch * rows, batch * rows))
+    g = None
+    try:
+        _put(ctx, dx, np.zeros((batch, cols)))
+        ctx.qmm_dev_noalloc(w, 0, dx, de, batch, 0)  # the kernels are loaded outside the capture
+        ctx.synchronize()
+        g = _Graph(ctx, lambda: ctx.qmm_dev_noalloc(w, 0, dx, dy, batch, 0))
+        for _ in range(4):
+            _put(ctx, dx, rng.standard_normal((batch, cols)))
+            g.launch()
+            ctx.qmm_dev_noalloc(w, 0, dx, de, batch, 0)
+            ctx.synchronize()
+            a, b = (d.to_numpy(np.uint32, batch * rows) for d in (dy, de))
+            assert np.array_equal(a, b)
+    finally:
+        if g:
+            g.free()
+        for h in (w, dx, dy, de):
+            h.free()
+
+
+@pytest.mark.parametrize("fmt,t", [(mm.Q8_0, 40), (mm.IQ2_XXS, 40), (mm.Q8_0, 9)])
+def test_moe_layer_under_capture(ctx, fmt, t):
+    """A captured layer call of several tokens (more than one routing workgroup
+    at 40) replayed with other tokens each time: the eager call's bits."""
+    rng = np.random.default_rng(980 + fmt + t)
+    hidden, inter, E = 512, 256, 12
+    layer = mm.MoeLayer(ctx, hidden=hidden, inter=inter, n_experts=E, expert_type=fmt,
+                        router=rng.normal(0.0, 0.05, (E, hidden)).astype(np.float32),
+                        gate=mm.make_weight(rng, fmt, inter, hidden, E), up=mm.make_weight(rng, fmt, inter, hidden, E),
+                        down=mm.make_weight(rng, fmt, hidden, inter, E),
+                        shared=tuple(mm.make_weight(rng, fmt, *s) for s in ((inter, hidden), (inter, hidden), (hidden, inter))),
+                        shared_inter=inter)
+    dx, dy, de = (mm.DeviceArray(ctx, t * hidden * 4) for _ in range(3))
+    g = None
+    try:
+        _put(ctx, dx, np.zeros((t, hidden)))
+        layer.ffn_dev(dx, de, t)  # the kernels are loaded outside the capture
+        ctx.synchronize()
+        g = _Graph(ctx, lambda: layer.ffn_dev(dx, dy, t))
+        for _ in range(4):
+            _put(ctx, dx, rng.standard_normal((t, hidden)))
+            g.launch()
+            layer.ffn_dev(dx, de, t)
+            ctx.synchronize()
+            a, b = (d.to_numpy(np.uint32, t * hidden) for d in (dy, de))
+            assert np.array_equal(a, b)
+    finally:
+        if g:
+            g.free()
+        layer.free()
+        for h in (dx, dy, de):
+            h.free()
