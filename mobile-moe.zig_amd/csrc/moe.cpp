@@ -31,7 +31,7 @@
 //   combine         weighted sum in route order + shared
 //                   + deferral bias                           "moe_combine"
 // No routing result returns to the host in between.
-#include <cmath>
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -217,49 +217,39 @@ int gemv_launch(mmhip_ctx* ctx, const mmhip_weight* w, const char* family, const
 
 int check_hip(hipError_t e, const char* what) { return e == hipSuccess ? MMHIP_OK : hip_fail(e, what); }
 
-// A separate shared expert of a call of several tokens: gate, up and the
-// activation in one dense launch, down in another (digits: five launches).
-bool shared_tile(const mmhip_moe_layer* L, uint32_t T) {
-    return T > 1 && L->sh_gu && gemm_tile_fits(L->sh_gu->geom, T, L->hidden) &&
-           gemm_tile_fits(L->sh_dn->geom, T, L->shared_inter);
-}
-
-// Whether a call of several tokens runs its routed experts on the bf16 matrix
-// cores. Q8_0 experts always (layer of 64 experts of 1536, hidden 2048: 2 tokens
-// 47.0 -> 32.3 us, 64 tokens 138 -> 91, 256 tokens 396 -> 188; with even routing
-// 17 to 64 tokens lose up to a tenth, with skewed routing they gain a quarter).
-//
-// An IQ2_XXS item costs more there than one on the digit kernel, but holds 16
-// rows instead of 8, saves the quantising launch and needs no large call. So the
-// digits stay where many experts get few rows each: where the call is large
-// enough for their 1024-thread workgroups, its experts' weights outweigh the
-// saved launch (matrices of 1.3 M weights and more, 52 M of them touched under even
-// routing) and an expert gets eight rows or fewer on average. How far the rows
-// spread is known on the device only, so the line was drawn for even routing and
-// for one skewed as 1 / rank. Digits and tile, us, hidden 2048 with a merged shared
-// expert:                                   even              skewed
-//   64 experts of 1536, 4 tokens        48.7    44.6      48.2    39.4
-//     16 tokens                         55.5    72.3      45.4    48.0
-//     64 tokens                         76.9   100.8      70.1    72.7
-//     256 tokens                       153.9   149.4     155.8   146.1
-//   24 experts of 1536, 32 tokens       52.8    57.9      50.8    54.6
-//   16 experts of 1536, 24 tokens       53.5    49.5      53.3    48.8
-//   64 experts of 768, 6 tokens         47.5    41.2      40.2    33.1
-//     32 tokens                         50.9    59.4      46.7    43.5
-//   64 experts of 512, 32 tokens        47.4    50.0      41.1    37.9
-// Over 11,520 calls (8 layer sizes, 16 to 128 experts, with every kind of shared
-// expert, 2 to 256 tokens, both routings) this line is within 0.8% of the faster
-// of the two on average; 87 calls are more than 3% slower than with digits alone.
-bool moe_tile(const mmhip_moe_layer* L, uint32_t T, uint32_t k, int num_cu) {
+// Whether a call of several tokens runs its experts on the bf16 matrix cores.
+// Q8_0 experts always (layer of 64 experts of 1536, hidden 2048: 2 tokens 47.0
+// -> 32.3 us, 64 tokens 138 -> 91, 256 tokens 396 -> 188). IQ2_XXS experts keep
+// the digit kernel's 8-row items where a large layer's call has enough of them
+// for its 1024-thread workgroups but so few tokens per expert that the 16-row
+// tile would be mostly empty rows. Digits and tile, us, hidden 2048 with a merged
+// shared expert:
+//   64 experts of 1536: 4 tokens (below those workgroups) 48.9 and 38.9, 16 tokens
+//     45.8 and 48.1, 64 tokens 69.9 and 71.7, 72 tokens 72.4 and 78.8, 96 tokens
+//     84.3 and 84.5, 256 tokens 155.7 and 144.7;
+//   24 experts of 1536: 40 tokens 57.4 and 59.8, 48 tokens 60.0 and 60.1, 72
+//     tokens 70.3 and 68.3; 16 experts get as many rows each sooner: 32 tokens
+//     52.1 and 49.7;
+//   48 experts of 1280: 52 tokens 58.5 and 63.1, 96 tokens 75.8 and 76.5, 128
+//     tokens 87.9 and 86.3;
+//   64 experts of 1024: 4 tokens 46.3 and 33.1 (32 experts), 28 tokens 47.0 and 42.4, 48
+//     tokens 52.6 and 57.1, 72 tokens 61.6 and 63.8, 128 tokens 81.5 and 79.2
+//   64 experts of 768: 4 tokens 43.0 and 32.2, 16 tokens 39.1 and 37.1, 48 tokens
+//     49.2 and 51.3, 128 tokens 71.6 and 70.6.
+// A separate shared expert costs the digit path five launches (92.5 us against
+// 80.1 at 64 tokens).
+bool moe_tile(const mmhip_moe_layer* L, uint32_t T, int num_cu) {
     if (T == 1) return false;
     const TileGeom& g = L->gu->geom;
-    const double size = (double)L->inter * L->hidden, E = L->n_experts;
-    const double touched = E * (1.0 - std::exp(-(double)k * T / E));  // experts, even routing
-    if (g.fmt == kFmtIq2 && size >= 1.3e6 && size * touched >= 52e6 && k * T <= 8 * L->n_experts &&
-        group_large(g, route_max_work(T, L->n_experts, kQmmTokens), num_cu))
+    const uint64_t size = (uint64_t)L->inter * L->hidden;
+    const uint32_t E = L->n_experts;
+    const uint32_t most = E >= 24 && size >= 5u << 19 ? std::max(E, std::min(2 * E, 96u)) : E;
+    if (g.fmt == kFmtIq2 && !L->sh_gu && T <= most && size >= 1u << 21 &&
+        group_large(g, route_max_work(T, E, kQmmTokens), num_cu))
         return false;
-    return gemm_tile_fits(L->gu->geom, T, L->hidden) && gemm_tile_fits(L->dn->geom, 5 * T, L->inter) &&
-           (!L->sh_gu || shared_tile(L, T));
+    if (!gemm_tile_fits(L->gu->geom, T, L->hidden) || !gemm_tile_fits(L->dn->geom, 5 * T, L->inter)) return false;
+    return !L->sh_gu || (gemm_tile_fits(L->sh_gu->geom, T, L->hidden) &&
+                         gemm_tile_fits(L->sh_dn->geom, T, L->shared_inter));
 }
 
 // The device sequence of one call; T in [1, kMaxTok].
@@ -294,7 +284,7 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
     r.n_work = L->n_work;
     r.inter = I;
     const bool fused = T == 1 && L->decode_fused;
-    const bool tile = moe_tile(L, T, k, ctx->num_cu);
+    const bool tile = moe_tile(L, T, ctx->num_cu);
     if (tile) {
         r.item_rows = kTileTokens;
         r.paired = 1;
@@ -310,11 +300,10 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
     }
     const bool sep_shared = L->has_shared && !L->shared_merged;
     const uint32_t SI = L->shared_inter;
-    const bool sh_tile = shared_tile(L, T);
     // One activation scale per 256 columns when an IQ2_XXS grouped matmul
     // reads the hidden digits (routed experts or the shared expert); then the
     // routing launch also quantises them.
-    const bool wide_h = L->gu->geom.fmt == kFmtIq2 || (sep_shared && !sh_tile && L->sh_gu->geom.fmt == kFmtIq2);
+    const bool wide_h = L->gu->geom.fmt == kFmtIq2 || (sep_shared && L->sh_gu->geom.fmt == kFmtIq2);
     const QuantAct qh = quant_act_view(L->xq_h, T, L->gu->geom.cols_pad);
     if (T > 1) {
         if (wide_h && !tile) {
@@ -327,16 +316,6 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
         TimedLaunch tl(ctx, "moe_route");
         MOE_TRY(check_hip(launch_route(r, s), "moe: route"));
     }
-    auto shared_gateup = [&] {
-        return check_hip(launch_gemm_tile(L->sh_gu->recs, L->sh_gu->dvals, L->sh_gu->geom, 0, true, hidden, H, T, L->y_sh,
-                                          SI, 1, ctx->num_cu, s),
-                         "moe: shared gate/up");
-    };
-    auto shared_down = [&] {
-        return check_hip(launch_gemm_tile(L->sh_dn->recs, L->sh_dn->dvals, L->sh_dn->geom, 0, false, L->y_sh, SI, T,
-                                          L->eo + 4 * (uint64_t)T * H, H, 1, ctx->num_cu, s),
-                         "moe: shared down");
-    };
     if (fused) {
         // Decode in one launch: router, routing, gate/up, down and combine.
         const TileGeom& gg = L->gu->geom;
@@ -417,14 +396,20 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
             MOE_TRY(check_hip(launch_gemm_tile_experts(L->gu->recs, L->gu->dvals, L->gu->geom, true, L->xp, H, T,
                                                        L->slot_tok, L->work_gu, L->n_work, items, T, L->y_gu, I, s),
                               "moe: gate/up"));
-            if (sh_tile) MOE_TRY(shared_gateup());
+            if (sep_shared)
+                MOE_TRY(check_hip(launch_gemm_tile(L->sh_gu->recs, L->sh_gu->dvals, L->sh_gu->geom, 0, true, hidden, H,
+                                                   T, L->y_sh, SI, 1, ctx->num_cu, s),
+                                  "moe: shared gate/up"));
         }
         {
             TimedLaunch tl(ctx, "moe_down");
             MOE_TRY(check_hip(launch_gemm_tile_experts(L->dn->recs, L->dn->dvals, L->dn->geom, false, L->y_gu, I, 5 * T,
                                                        nullptr, L->work_dn, L->n_work + 1, items, T, L->eo, H, s),
                               "moe: down"));
-            if (sh_tile) MOE_TRY(shared_down());
+            if (sep_shared)
+                MOE_TRY(check_hip(launch_gemm_tile(L->sh_dn->recs, L->sh_dn->dvals, L->sh_dn->geom, 0, false, L->y_sh,
+                                                   SI, T, L->eo + 4 * (uint64_t)T * H, H, 1, ctx->num_cu, s),
+                                  "moe: shared down"));
         }
     } else {
         const TileGeom& gg = L->gu->geom;
@@ -438,9 +423,7 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
             MOE_TRY(check_hip(launch_group_experts(L->gu->recs, L->gu->dvals, gg, qh, L->slot_tok, L->work_gu, L->n_work,
                                                    route_max_work(T, E, kQmmTokens), L->y_gu, 2 * (uint64_t)I, ctx->num_cu, s),
                               "moe: gate/up"));
-            if (sh_tile) {
-                MOE_TRY(shared_gateup());
-            } else if (sep_shared) {
+            if (sep_shared) {
                 const TileGeom& gs = L->sh_gu->geom;
                 if (gs.cols_pad != gg.cols_pad) {
                     set_error(MMHIP_ERR_UNSUPPORTED, "moe: shared gate/up padding differs from the routed experts'");
@@ -466,9 +449,7 @@ int ffn_enqueue(mmhip_ctx* ctx, mmhip_moe_layer* L, const float* hidden, float* 
             MOE_TRY(check_hip(launch_group_experts(L->dn->recs, L->dn->dvals, gd, qd, nullptr, L->work_dn, L->n_work + 1,
                                                    route_max_work(T, E, kQmmTokens) / 2, L->eo, H, ctx->num_cu, s),
                               "moe: down"));
-            if (sh_tile) {
-                MOE_TRY(shared_down());
-            } else if (sep_shared) {
+            if (sep_shared) {
                 const TileGeom& gs = L->sh_dn->geom;
                 const QuantAct qs = quant_act_view(L->xq_sd, T, gs.cols_pad);
                 MOE_TRY(check_hip(launch_quantize_silu(L->y_sh, 2 * (uint64_t)SI, SI, nullptr, T, SI,
