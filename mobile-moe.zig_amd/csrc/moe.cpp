@@ -31,7 +31,6 @@
 //   combine         weighted sum in route order + shared
 //                   + deferral bias                           "moe_combine"
 // No routing result returns to the host in between.
-#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -221,31 +220,18 @@ int check_hip(hipError_t e, const char* what) { return e == hipSuccess ? MMHIP_O
 // Q8_0 experts always (layer of 64 experts of 1536, hidden 2048: 2 tokens 47.0
 // -> 32.3 us, 64 tokens 138 -> 91, 256 tokens 396 -> 188). IQ2_XXS experts keep
 // the digit kernel's 8-row items where a large layer's call has enough of them
-// for its 1024-thread workgroups but so few tokens per expert that the 16-row
-// tile would be mostly empty rows. Digits and tile, us, hidden 2048 with a merged
-// shared expert:
-//   64 experts of 1536: 4 tokens (below those workgroups) 48.9 and 38.9, 16 tokens
-//     45.8 and 48.1, 64 tokens 69.9 and 71.7, 72 tokens 72.4 and 78.8, 96 tokens
-//     84.3 and 84.5, 256 tokens 155.7 and 144.7;
-//   24 experts of 1536: 40 tokens 57.4 and 59.8, 48 tokens 60.0 and 60.1, 72
-//     tokens 70.3 and 68.3; 16 experts get as many rows each sooner: 32 tokens
-//     52.1 and 49.7;
-//   48 experts of 1280: 52 tokens 58.5 and 63.1, 96 tokens 75.8 and 76.5, 128
-//     tokens 87.9 and 86.3;
-//   64 experts of 1024: 4 tokens 46.3 and 33.1 (32 experts), 28 tokens 47.0 and 42.4, 48
-//     tokens 52.6 and 57.1, 72 tokens 61.6 and 63.8, 128 tokens 81.5 and 79.2
-//   64 experts of 768: 4 tokens 43.0 and 32.2, 16 tokens 39.1 and 37.1, 48 tokens
-//     49.2 and 51.3, 128 tokens 71.6 and 70.6.
-// A separate shared expert costs the digit path five launches (92.5 us against
-// 80.1 at 64 tokens).
+// for its 1024-thread workgroups but no more tokens than experts, so that the
+// 16-row tile would be mostly empty rows (same layer, 16 tokens 46.7 us against
+// 48.0, 48 tokens 62.6 against 66.6, 64 tokens 70.6 against 71.4 to 73.2, 96
+// tokens 86.0 against 84.6, 256 tokens 158 against 147; 4 tokens, below those
+// workgroups, 49.2 against 39.1; hidden 1024, experts of 512: 64 tokens 39.3 against 31.0). A
+// separate shared expert costs the digit path five launches (92.6 us against
+// 79.6 at 64 tokens).
 bool moe_tile(const mmhip_moe_layer* L, uint32_t T, int num_cu) {
     if (T == 1) return false;
     const TileGeom& g = L->gu->geom;
-    const uint64_t size = (uint64_t)L->inter * L->hidden;
-    const uint32_t E = L->n_experts;
-    const uint32_t most = E >= 24 && size >= 5u << 19 ? std::max(E, std::min(2 * E, 96u)) : E;
-    if (g.fmt == kFmtIq2 && !L->sh_gu && T <= most && size >= 1u << 21 &&
-        group_large(g, route_max_work(T, E, kQmmTokens), num_cu))
+    if (g.fmt == kFmtIq2 && !L->sh_gu && T <= L->n_experts && (uint64_t)L->inter * L->hidden >= (1u << 21) &&
+        group_large(g, route_max_work(T, L->n_experts, kQmmTokens), num_cu))
         return false;
     if (!gemm_tile_fits(L->gu->geom, T, L->hidden) || !gemm_tile_fits(L->dn->geom, 5 * T, L->inter)) return false;
     return !L->sh_gu || (gemm_tile_fits(L->sh_gu->geom, T, L->hidden) &&

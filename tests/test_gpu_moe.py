@@ -216,14 +216,11 @@ def test_q8_expert_groups(ctx, orc, t, hidden, inter, variant):
         gpu.free()
 
 
-@pytest.mark.parametrize("t,n_exp,inter", [(15, 64, 1024), (16, 12, 1024), (40, 64, 1024), (40, 33, 1024),
-                                           (24, 23, 1280), (23, 23, 1280), (48, 24, 1280), (49, 24, 1280),
-                                           (97, 50, 1280)])
-def test_iq2_expert_groups_large_layer(ctx, orc, t, n_exp, inter):
-    """A layer large enough that calls of few tokens per expert keep the digit
-    kernel's items: both sides of that rule at every line it has, no shared
-    expert."""
-    hidden = 2048
+@pytest.mark.parametrize("t,n_exp", [(15, 64), (16, 12), (40, 64), (40, 33)])
+def test_iq2_expert_groups_large_layer(ctx, orc, t, n_exp):
+    """A layer large enough that calls of fewer tokens than experts keep the
+    digit kernel's items: both sides of that rule, no shared expert."""
+    hidden, inter = 2048, 1024
     rng = np.random.default_rng(380 + t + n_exp)
     w = _weights(rng, mm.IQ2_XXS, hidden, inter, n_exp, router_sigma=0.03)
     gpu, cpu = _layers(ctx, orc, mm.IQ2_XXS, hidden, inter, n_exp, *w)
