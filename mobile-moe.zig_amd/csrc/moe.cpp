@@ -224,9 +224,16 @@ int check_hip(hipError_t e, const char* what) { return e == hipSuccess ? MMHIP_O
 // 16-row tile would be mostly empty rows (same layer, 16 tokens 46.7 us against
 // 48.0, 48 tokens 62.6 against 66.6, 64 tokens 70.6 against 71.4 to 73.2, 96
 // tokens 86.0 against 84.6, 256 tokens 158 against 147; 4 tokens, below those
-// workgroups, 49.2 against 39.1; hidden 1024, experts of 512: 64 tokens 39.3 against 31.0). A
-// separate shared expert costs the digit path five launches (92.6 us against
-// 79.6 at 64 tokens).
+// workgroups, 49.2 against 39.1; hidden 1024, experts of 512: 64 tokens 39.3 against
+// 31.0; experts of 1024 with hidden 2048, the smallest on this side: 28 tokens 47.0
+// against 42.4, 48 tokens 52.6 against 57.1). A separate shared expert costs the
+// digit path five launches (92.6 us against 79.6 at 64 tokens).
+//
+// These were routed as skewed as 1 / rank. Routed evenly, more experts get fewer
+// rows each, and the digits end first over a wider range: 64 experts of 768, 32
+// tokens 50.9 against 59.4 us, 24 experts of 1536, 32 tokens 52.8 against 57.9,
+// 128 experts of 768, 32 tokens 62.0 against 77.9. Those calls stay on the tile
+// kernel for its precision: 4e-6 of the result where the digits give 8e-5.
 bool moe_tile(const mmhip_moe_layer* L, uint32_t T, int num_cu) {
     if (T == 1) return false;
     const TileGeom& g = L->gu->geom;
